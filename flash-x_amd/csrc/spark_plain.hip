@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
 #pragma unroll
         for (int q = -R; q <= R; q++) cur[q + 2] = ud[q + 2] * cur[q + 2];
       }
-      recon1<RECON>(cur, fl_c, up, um);
+      recon1_short<RECON>(cur, fl_c, up, um);
       sm[v * NT + tid] = up;
       umr[v] = um;
       if (v == R_DENS) sm[(R_NUM + 0) * NT + tid] = cur[2];
@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
           for (int q = 0; q < 5; q++) cur[q] = nxt[q];
           if (v + 1 < NSM) stencil(R_NUM + v + 1, nxt);
           __builtin_amdgcn_sched_barrier(0);
-          recon1<RECON>(cur, fl_c, up, um);
+          recon1_short<RECON>(cur, fl_c, up, um);
           sm[v * NT + tid] = up;
           ums[v] = um;
         }

@@ -321,3 +321,23 @@ def test_fp32_flux_100_steps_mixed_blocks_vs_fp64():
     assert cnt[0] == 0
     assert nm["rho"][0] <= 1e-5
     assert nm["E"][0] <= 1e-5
+
+
+def test_plain_short_quotients_equal_ieee_divides():
+    """The plain form's WENO5 takes short quotients where a wave's smoothness
+    indicators are below 2^900 and IEEE divides elsewhere; the batched FP64
+    form always takes the IEEE divides, so the two must agree bit for bit with
+    scalars whose indicators are far below the 1e-36 added to them, ordinary,
+    near the range's end on both sides, and beyond it (where the weights
+    overflow to the same NaN)."""
+    scales = (1e-170, 1.0, 1e100, 2.0 ** 448, 2.0 ** 452, 1e145)
+    prob = problems.batched(nblocks=6, nguard=10, sizes=(8, 16), probs=(0.5, 0.5), shock_every=2, nscalars=len(scales))
+    r = np.random.default_rng(5)
+    for a in prob.arrays:
+        for q, s in enumerate(scales):
+            a[..., capi.SPARK_NPROP + q] = s * (1.0 + 0.5 * r.random(a.shape[:-1]))
+    res = [run_gpu(prob, 2, form) for form in ("plain_fp64", "batched_fp64")]
+    assert np.array_equal(res[0][0], res[1][0])
+    for x, y in zip(interiors(prob, res[0][1]), interiors(prob, res[1][1])):
+        assert np.array_equal(x, y, equal_nan=True)
+        assert np.isfinite(x[..., : capi.SPARK_NPROP + 4]).all()
