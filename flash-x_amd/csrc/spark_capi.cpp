@@ -18,6 +18,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <string>
 #include <tuple>
@@ -27,6 +28,7 @@
 #include "spark_batched.hpp"
 #include "spark_regions.hpp"
 #include "spark_launch.hpp"
+#include "spark_transfer.hpp"
 
 using spark::BlockMeta;
 using spark::DevParams;
@@ -826,6 +828,7 @@ int spark_init(int device) {
 int spark_finalize(void) {
   if (g_stream) {
     HIPCHK(hipStreamSynchronize(g_stream));
+    spark::xfer_release();
     HIPCHK(hipStreamDestroy(g_stream));
   }
   g_stream = nullptr;
@@ -1046,13 +1049,13 @@ int spark_batch_destroy(spark_batch* b) {
   return SPARK_OK;
 }
 
-// AoS <-> SoA transfer in rounds of blocks through a device staging area of
-// `cap` doubles (`stage`), with device room for `maxb` block offsets
-// (`off_d`) and the variable map (`vidx_d`); off_h is host room for maxb
-// offsets.  Every round ends with the stream synchronised, so the staging
-// area is free again when the next round writes it.
-static int transfer_rounds(spark_batch* b, double* const* host, int to_device, int interior_only, double* pool,
-                           double* stage, int64_t cap, int64_t* off_d, int* vidx_d, int maxb, int64_t* off_h) {
+// AoS -> SoA in rounds of blocks through a fixed device staging area of `cap`
+// doubles (`stage`), with device room for `maxb` block offsets (`off_d`) and
+// the variable map (`vidx_d`); off_h is host room for maxb offsets.  Every
+// round ends with the stream synchronised, so the staging area is free again
+// when the next round writes it.
+static int pack_rounds(spark_batch* b, const double* const* host, double* stage, int64_t cap, int64_t* off_d,
+                       int* vidx_d, int maxb, int64_t* off_h) {
   const int nunk = b->p.nunk_vars;
   HIPCHK(hipMemcpy(vidx_d, b->p.var_index, sizeof(int) * b->nvar, hipMemcpyHostToDevice));
   int rc = SPARK_OK;
@@ -1072,54 +1075,33 @@ static int transfer_rounds(spark_batch* b, double* const* host, int to_device, i
     for (int i = i0; i < i1 && e == hipSuccess; i++) {
       const BlockMeta& m = b->meta_h[i];
       const int64_t sz = (int64_t)nunk * m.NX * m.NY * m.NZ;
-      // unpack also stages the host block first, so unk slots outside the
-      // variable map (and guards when interior_only) keep their host values
       e = hipMemcpy(stage + off_h[i - i0], host[i], sizeof(double) * sz, hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) {
-      if (to_device)
-        e = spark::plain_aos_to_soa(g_stream, b->meta_d + i0, i1 - i0, (int)b->max_cells, stage, off_d, nunk, vidx_d,
-                                    b->nvar, pool);
-      else
-        e = spark::plain_soa_to_aos(g_stream, b->dp, b->meta_d + i0, i1 - i0, (int)b->max_cells, pool, stage, off_d,
-                                    nunk, vidx_d, b->nvar, interior_only);
-    }
+    if (e == hipSuccess)
+      e = spark::plain_aos_to_soa(g_stream, b->meta_d + i0, i1 - i0, (int)b->max_cells, stage, off_d, nunk, vidx_d,
+                                  b->nvar, b->U);
     if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-    for (int i = i0; i < i1 && e == hipSuccess && !to_device; i++) {
-      const BlockMeta& m = b->meta_h[i];
-      const int64_t sz = (int64_t)nunk * m.NX * m.NY * m.NZ;
-      e = hipMemcpy(host[i], stage + off_h[i - i0], sizeof(double) * sz, hipMemcpyDeviceToHost);
-    }
-    if (e != hipSuccess) rc = fail(SPARK_ERR_HIP, "pack/unpack: %s", hipGetErrorString(e));
+    if (e != hipSuccess) rc = fail(SPARK_ERR_HIP, "pack: %s", hipGetErrorString(e));
     i0 = i1;
   }
   return rc;
 }
 
-static int transfer(spark_batch* b, double* const* host, int to_device, int interior_only, double* pool) {
-  const int nunk = b->p.nunk_vars;
-  // stage at most ~256 MiB of AoS data per round trip
-  const int64_t cap = std::max<int64_t>((int64_t)nunk * b->max_cells, (int64_t)32 << 20);
-  double* stage = nullptr;
-  int64_t* off_d = nullptr;
-  int* vidx_d = nullptr;
-  HIPCHK(hipMalloc((void**)&stage, sizeof(double) * cap));
-  HIPCHK(hipMalloc((void**)&off_d, sizeof(int64_t) * b->nblk));
-  HIPCHK(hipMalloc((void**)&vidx_d, sizeof(int) * b->nvar));
-  std::vector<int64_t> off_h(b->nblk);
-  const int rc = transfer_rounds(b, host, to_device, interior_only, pool, stage, cap, off_d, vidx_d, b->nblk,
-                                 off_h.data());
-  (void)hipFree(stage);
-  (void)hipFree(off_d);
-  (void)hipFree(vidx_d);
-  return rc;
+static spark::XferJob xfer_job(spark_batch* b, double* pool, int interior_only) {
+  return spark::XferJob{b->meta_h.data(), b->meta_d, b->nblk, b->p.nguard, b->p.ndim, b->nvar, b->p.nunk_vars,
+                        b->p.var_index, pool, interior_only};
 }
 
 int spark_pack(spark_batch* b, const double* const* unk_blocks) {
   if (!b || !unk_blocks) return fail(SPARK_ERR_ARG, "spark_pack: null argument");
   for (int i = 0; i < b->nblk; i++)
     if (!unk_blocks[i]) return fail(SPARK_ERR_ARG, "spark_pack: block %d pointer is null", i);
-  return transfer(b, const_cast<double* const*>(unk_blocks), 1, 0, b->U);
+  try {
+    HIPCHK(spark::xfer_pack(xfer_job(b, b->U, 0), unk_blocks, g_device, g_stream));
+  } catch (const std::exception& e) {
+    return fail(SPARK_ERR_HIP, "spark_pack: %s", e.what());
+  }
+  return SPARK_OK;
 }
 
 int spark_pack_noalloc(spark_batch* b, const double* const* unk_blocks) {
@@ -1139,18 +1121,21 @@ int spark_pack_noalloc(spark_batch* b, const double* const* unk_blocks) {
   }
   unsigned char* area = static_cast<unsigned char*>(g_noalloc[g_device]);
   int64_t off_h[spark::NOALLOC_MAXB];
-  return transfer_rounds(b, const_cast<double* const*>(unk_blocks), 1, 0, b->U,
-                         reinterpret_cast<double*>(area + spark::NOALLOC_STAGE), cap,
-                         reinterpret_cast<int64_t*>(area + 256), reinterpret_cast<int*>(area), spark::NOALLOC_MAXB,
-                         off_h);
+  return pack_rounds(b, unk_blocks, reinterpret_cast<double*>(area + spark::NOALLOC_STAGE), cap,
+                     reinterpret_cast<int64_t*>(area + 256), reinterpret_cast<int*>(area), spark::NOALLOC_MAXB, off_h);
 }
 
 int spark_unpack(spark_batch* b, double* const* unk_blocks, int interior_only, int which) {
   if (!b || !unk_blocks) return fail(SPARK_ERR_ARG, "spark_unpack: null argument");
   for (int i = 0; i < b->nblk; i++)
     if (!unk_blocks[i]) return fail(SPARK_ERR_ARG, "spark_unpack: block %d pointer is null", i);
-  HIPCHK(hipStreamSynchronize(g_stream));
-  return transfer(b, unk_blocks, 0, interior_only, which ? (b->star ? b->star : b->S) : b->U);
+  double* pool = which ? (b->star ? b->star : b->S) : b->U;
+  try {
+    HIPCHK(spark::xfer_unpack(xfer_job(b, pool, interior_only != 0), unk_blocks, g_device, g_stream));
+  } catch (const std::exception& e) {
+    return fail(SPARK_ERR_HIP, "spark_unpack: %s", e.what());
+  }
+  return SPARK_OK;
 }
 
 int spark_set_uniform_grid(spark_batch* b, int nbx, int nby, int nbz) {

@@ -104,9 +104,6 @@ hipError_t amr_fill(const PlainLaunch& L, const AmrGrid& G, double* U, const Var
 hipError_t amr_flux_exchange(const PlainLaunch& L, const AmrGrid& G, double* const fb[3], double* const fc[3]);
 hipError_t plain_aos_to_soa(hipStream_t st, const BlockMeta* meta, int nblk, int maxcells, const double* aos,
                             const int64_t* aos_off, int nunk, const int* var_index, int nvar, double* U);
-hipError_t plain_soa_to_aos(hipStream_t st, const DevParams& P, const BlockMeta* meta, int nblk, int maxcells,
-                            const double* U, double* aos, const int64_t* aos_off, int nunk, const int* var_index,
-                            int nvar, int interior);
 
 // fixed staging area of spark_pack_noalloc (spark_noalloc.hip): 64 MiB per
 // device, of which the AoS staging of one round of blocks starts at

@@ -963,8 +963,8 @@ __global__ void __launch_bounds__(256) k_correct(DevParams P, const BlockMeta* _
 }
 
 // ---------------------------------------------------------------------------
-// AoS (unk: variable fastest, host-packed into a contiguous staging buffer)
-// <-> SoA transposes.  var_index[v] gives the unk slot of canonical var v.
+// AoS (unk: variable fastest, in the fixed staging area of spark_pack_noalloc)
+// -> SoA transpose.  var_index[v] gives the unk slot of canonical var v.
 __global__ void __launch_bounds__(256) k_aos_to_soa(const BlockMeta* __restrict__ meta, const double* __restrict__ aos,
                                                     const int64_t* __restrict__ aos_off, int nunk,
                                                     const int* __restrict__ var_index, int nvar,
@@ -974,23 +974,6 @@ __global__ void __launch_bounds__(256) k_aos_to_soa(const BlockMeta* __restrict_
   const double* src = aos + aos_off[blockIdx.y];
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x)
     for (int v = 0; v < nvar; v++) U[m.base + v * m.cstride + t] = src[(int64_t)t * nunk + var_index[v]];
-}
-
-__global__ void __launch_bounds__(256) k_soa_to_aos(DevParams P, const BlockMeta* __restrict__ meta,
-                                                    const double* __restrict__ U, double* __restrict__ aos,
-                                                    const int64_t* __restrict__ aos_off, int nunk,
-                                                    const int* __restrict__ var_index, int nvar, int interior) {
-  const BlockMeta m = meta[blockIdx.y];
-  const int total = m.NX * m.NY * m.NZ;
-  double* dst = aos + aos_off[blockIdx.y];
-  Lims L = stage_lims(P, m, 0);
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
-    if (interior) {
-      const int i = t % m.NX, j = (t / m.NX) % m.NY, k = t / (m.NX * m.NY);
-      if (i < L.lo[0] || i > L.hi[0] || j < L.lo[1] || j > L.hi[1] || k < L.lo[2] || k > L.hi[2]) continue;
-    }
-    for (int v = 0; v < nvar; v++) dst[(int64_t)t * nunk + var_index[v]] = U[m.base + v * m.cstride + t];
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1276,14 +1259,6 @@ hipError_t plain_aos_to_soa(hipStream_t st, const BlockMeta* meta, int nblk, int
                             const int64_t* aos_off, int nunk, const int* var_index, int nvar, double* U) {
   hipLaunchKernelGGL(k_aos_to_soa, dim3(grid_x_for(maxcells, 512), nblk), dim3(256), 0, st, meta, aos, aos_off, nunk,
                      var_index, nvar, U);
-  return hipGetLastError();
-}
-
-hipError_t plain_soa_to_aos(hipStream_t st, const DevParams& P, const BlockMeta* meta, int nblk, int maxcells,
-                            const double* U, double* aos, const int64_t* aos_off, int nunk, const int* var_index,
-                            int nvar, int interior) {
-  hipLaunchKernelGGL(k_soa_to_aos, dim3(grid_x_for(maxcells, 512), nblk), dim3(256), 0, st, P, meta, U, aos, aos_off,
-                     nunk, var_index, nvar, interior);
   return hipGetLastError();
 }
 

@@ -121,7 +121,11 @@ int spark_batch_destroy(spark_batch* b);
 
 /* Host unk blocks (guard-celled box, nunk_vars fastest) -> device.
  * Replaces: tileDesc%getDataPtr + saveState's read of Uin,
- * Grid_tile.F90:157-267 and Spark/Hydro_funcs.F90-mc:512-541. */
+ * Grid_tile.F90:157-267 and Spark/Hydro_funcs.F90-mc:512-541.
+ * pack and unpack stage through 4 x 8 MiB of pinned host and of device
+ * memory that the library keeps from its first transfer to spark_finalize
+ * (transfers of several threads take turns); from 4 MiB on, three helper
+ * threads share the host copies for the length of the call. */
 int spark_pack(spark_batch* b, const double* const* unk_blocks);
 /* spark_pack without device allocation.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (tight stepping
@@ -134,7 +138,8 @@ int spark_pack(spark_batch* b, const double* const* unk_blocks);
  * threads) race. */
 int spark_pack_noalloc(spark_batch* b, const double* const* unk_blocks);
 /* Device -> host unk blocks; interior_only mirrors updateState
- * (Spark/Hydro_funcs.F90-mc:573-574).  which = 0: solution, 1: the stage
+ * (Spark/Hydro_funcs.F90-mc:573-574) and writes only the interior cells;
+ * unk slots outside the variable map keep their host values.  which = 0: solution, 1: the stage
  * state (hy_starState) written by the last stage run before a step's final
  * stage. */
 int spark_unpack(spark_batch* b, double* const* unk_blocks, int interior_only, int which);
