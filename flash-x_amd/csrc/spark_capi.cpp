@@ -122,6 +122,20 @@ struct spark_batch {
   bool dt_control = false;
   int amr_remap_count = 0;
   int amr_partial_count = 0;
+  // plain form on a block hierarchy: per stage the boxes its sweeps run, one
+  // group per box shape (plain_groups_build); the guard sectors a block takes
+  // from same-level leaves between the stages, and the blocks with some but
+  // not all of them
+  struct PlainGroup {
+    int ext[3];
+    int n;
+    bool interior;  // holds the blocks' interiors: accumulates the flux registers
+    int* ids_d;
+    int* lo_d;
+  };
+  std::vector<PlainGroup> groups[3];
+  uint32_t* amr_nmask_d = nullptr;
+  int* partial_ids_d = nullptr;
   bool same_level = true;      // SPARK_OPT_SAME_LEVEL_HALOS
   int* remap_ids_d = nullptr;  // the remapping blocks
   int* tele_ids_d = nullptr;   // the telescoping blocks
@@ -195,6 +209,8 @@ PlainLaunch make_launch(spark_batch* b, const ShapeClass& c) {
   L.blist = c.ids_d;
   L.nblk = (int)c.ids.size();
   L.nx = c.nx; L.ny = c.ny; L.nz = c.nz;
+  L.blo = nullptr;
+  L.ext[0] = L.ext[1] = L.ext[2] = 0;
   L.U0 = b->U;
   L.Sin = b->S;
   L.Sout = b->S;
@@ -225,7 +241,29 @@ void drop_graph(spark_batch* b);
 
 // batched forms on a block hierarchy: same-level halos in use
 bool amr_remap_on(const spark_batch* b) {
-  return b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
+  return b->fused && b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
+}
+
+// plain form on a block hierarchy: the guard sectors across which lies a leaf
+// of the block's own level are copied from that leaf between the stages, and
+// a block computes only its interior and the other sectors.  The values are
+// those of telescoping (the same cells from the same inputs).
+bool plain_same_level(const spark_batch* b) {
+  return b->amr && !b->fused && b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
+}
+
+void free_plain_groups(spark_batch* b) {
+  for (auto& st : b->groups) {
+    for (auto& g : st) {
+      if (g.ids_d) (void)hipFree(g.ids_d);
+      if (g.lo_d) (void)hipFree(g.lo_d);
+    }
+    st.clear();
+  }
+  if (b->amr_nmask_d) (void)hipFree(b->amr_nmask_d);
+  if (b->partial_ids_d) (void)hipFree(b->partial_ids_d);
+  b->amr_nmask_d = nullptr;
+  b->partial_ids_d = nullptr;
 }
 
 int run_dt(spark_batch* b, int hist_slot) {
@@ -240,6 +278,10 @@ int run_dt(spark_batch* b, int hist_slot) {
                                hist_slot >= 0 && b->dt_control ? b->dtctl_d : nullptr));
   return SPARK_OK;
 }
+
+// layers around the interior that a stage of it and the step's shock
+// detection (hybrid solver: of the layer around it too) read
+int interior_reach(const spark_batch* b) { return std::max(b->p.nstencil, b->p.use_hybrid_riemann ? 2 : 1); }
 
 // Guard fill of a uniform block grid.  full: every variable over every
 // guard layer (Grid_fillGuardCells semantics).  Otherwise only what the
@@ -273,6 +315,19 @@ int run_fill(spark_batch* b, double* pool, bool full, int depth) {
       L.blist = b->tele_ids_d;
       L.nblk = b->n_tele;
       HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth, b->p.use_hybrid_riemann ? nullptr : b->amr_smask_d, 1));
+    }
+  } else if (b->amr && !full && plain_same_level(b)) {
+    // blocks with same-level leaves all around: the layers stage 1 of the
+    // interior reads; the others to the depth they telescope from
+    if (b->amr_remap_count > 0) {
+      L.blist = b->remap_ids_d;
+      L.nblk = b->amr_remap_count;
+      HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, interior_reach(b)));
+    }
+    if (b->n_tele > 0) {
+      L.blist = b->tele_ids_d;
+      L.nblk = b->n_tele;
+      HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth));
     }
   } else if (b->amr) {
     HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth));
@@ -336,7 +391,7 @@ int stage1_reach(const spark_batch* b) {
   return (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + b->p.nstencil;
 }
 
-int run_step_begin(spark_batch* b) {
+int run_step_begin(spark_batch* b, bool same_level = false) {
   // SHOK over the cells the stages' hybrid Riemann solves read: the stage-1
   // region plus one layer (the reference computes NGUARD-1 layers; the
   // outer layers are never read before the next refill).  Without the
@@ -347,7 +402,19 @@ int run_step_begin(spark_batch* b) {
   // own in the stages) get it one layer out.
   const bool hyb = b->p.use_hybrid_riemann != 0;
   const int band = !hyb ? 0 : (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + 1;
-  if (amr_remap_on(b)) {
+  if (same_level && plain_same_level(b)) {
+    PlainLaunch L = make_launch(b, b->classes[0]);
+    if (b->n_tele > 0) {
+      L.blist = b->tele_ids_d;
+      L.nblk = b->n_tele;
+      HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, band));
+    }
+    if (b->amr_remap_count > 0) {
+      L.blist = b->remap_ids_d;
+      L.nblk = b->amr_remap_count;
+      HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, hyb ? 1 : 0));
+    }
+  } else if (amr_remap_on(b)) {
     // a hierarchy has one block shape
     PlainLaunch L = make_launch(b, b->classes[0]);
     if (b->n_tele > 0) {
@@ -484,6 +551,47 @@ int run_stage(spark_batch* b, int stage, int ngoff) {
   return SPARK_OK;
 }
 
+// one stage of the plain form over the boxes of its groups, then the guard
+// sectors the next stage reads from same-level leaves, copied from them
+int run_stage_groups(spark_batch* b, int stage) {
+  const double* co = b->coeff[stage - 1];
+  double* out = stage_out(b, stage);
+  if (stage != b->last_stage) b->star = out;
+  PlainLaunch L = make_launch(b, b->classes[0]);
+  L.weight = b->weights[stage - 1];
+  L.add_flux = stage > 1;
+  L.Sin = stage_in(b, stage);
+  L.Sout = out;
+  for (const auto& g : b->groups[stage - 1]) {
+    PlainLaunch G = L;
+    G.blist = g.ids_d;
+    G.blo = g.lo_d;
+    G.nblk = g.n;
+    for (int d = 0; d < 3; d++) {
+      G.ext[d] = g.ext[d];
+      if (!g.interior) G.fb[d] = nullptr;
+    }
+    HIPCHK(spark::plain_stage(G, 0, co[0], co[1], co[2], stage == b->last_stage));
+  }
+  if (stage == b->last_stage) return SPARK_OK;
+  spark::VarList vl;
+  vl.n = 0;
+  const int need[7] = {spark::V_DENS, spark::V_EINT, spark::V_GAMC, spark::V_PRES, spark::V_VELX, spark::V_VELY, spark::V_VELZ};
+  for (int v : need) vl.v[vl.n++] = v;
+  for (int s = 0; s < b->p.nscalars; s++) vl.v[vl.n++] = spark::V_NPROP + s;
+  if (b->amr_remap_count > 0) {
+    L.blist = b->remap_ids_d;
+    L.nblk = b->amr_remap_count;
+    HIPCHK(spark::amr_fill(L, b->amr_g, out, vl, b->p.nstencil));
+  }
+  if (b->amr_partial_count > 0) {
+    L.blist = b->partial_ids_d;
+    L.nblk = b->amr_partial_count;
+    HIPCHK(spark::amr_fill(L, b->amr_g, out, vl, b->limits_array[stage] + b->p.nstencil, b->amr_nmask_d, 0));
+  }
+  return SPARK_OK;
+}
+
 int run_step_end(spark_batch* b) {
   b->step_open = false;
   return SPARK_OK;
@@ -491,7 +599,12 @@ int run_step_end(spark_batch* b) {
 
 int run_full_step(spark_batch* b) {
   int rc;
-  if ((rc = run_step_begin(b))) return rc;
+  if ((rc = run_step_begin(b, true))) return rc;
+  if (plain_same_level(b)) {
+    for (int s = 1; s <= b->last_stage; s++)
+      if ((rc = run_stage_groups(b, s))) return rc;
+    return run_step_end(b);
+  }
   const bool refill = b->p.guard_mode == SPARK_GUARD_REFILL;
   for (int s = 1; s <= b->last_stage; s++) {
     if ((rc = run_stage(b, s, refill ? 0 : b->limits_array[s - 1]))) return rc;
@@ -515,6 +628,7 @@ void free_batch(spark_batch* b) {
   if (b->corr_ids_d) (void)hipFree(b->corr_ids_d);
   if (b->amr_map_d) (void)hipFree(b->amr_map_d);
   if (b->amr_org_d) (void)hipFree(b->amr_org_d);
+  free_plain_groups(b);
   for (int d = 0; d < 3; d++)
     if (b->fc[d]) (void)hipFree(b->fc[d]);
   for (auto& pl : b->plan) {
@@ -754,6 +868,58 @@ int fused_plan(spark_batch* b) {
   for (int s = 1; s <= b->last_stage; s++)
     if ((rc = build_stage_plan(b, s, nullptr, -1))) return rc;
   b->planned = true;
+  return SPARK_OK;
+}
+
+// The plain form's stage boxes on a hierarchy.  Every block's interior is one
+// group (full telescoping boxes of the blocks without a same-level leaf
+// around are another); the computed sectors of the others beside it are a
+// group per box shape.
+int plain_groups_build(spark_batch* b) {
+  free_plain_groups(b);
+  const int g = b->p.nguard;
+  const uint32_t all_sectors = ((1u << 27) - 1) & ~(1u << 13);
+  auto upload = [](int** dst, const std::vector<int>& v) -> hipError_t {
+    hipError_t e = hipMalloc((void**)dst, sizeof(int) * std::max<size_t>(1, v.size()));
+    return e == hipSuccess ? hipMemcpy(*dst, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice) : e;
+  };
+  for (int s = 1; s <= b->last_stage; s++) {
+    const int e = stage_ngoff(b, s);
+    struct Host { std::vector<int> ids, lo; };
+    std::map<std::tuple<int, int, int, bool>, Host> by;
+    for (int i = 0; i < b->nblk; i++) {
+      const BlockMeta& m = b->meta_h[i];
+      auto add = [&](const spark::Box& r, bool interior) {
+        Host& h = by[std::make_tuple(r.x1 - r.x0 + 1, r.y1 - r.y0 + 1, r.z1 - r.z0 + 1, interior)];
+        h.ids.push_back(i);
+        for (int q : {r.x0, r.y0, r.z0}) h.lo.push_back(q);
+      };
+      if (b->amr_remap_blk[i] == 0) {
+        add(region_box(m, g, e), true);
+        continue;
+      }
+      add(region_box(m, g, 0), true);
+      std::vector<Box> out;
+      if (b->amr_remap_blk[i] == 2) spark::outer_boxes(m.nx, m.ny, m.nz, g, e, b->amr_local[i], out);
+      for (const auto& r : out) add(r, false);
+    }
+    for (auto& kv : by) {
+      b->groups[s - 1].push_back(spark_batch::PlainGroup{{std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first)},
+                                                         (int)kv.second.ids.size(), std::get<3>(kv.first), nullptr, nullptr});
+      auto& gr = b->groups[s - 1].back();
+      HIPCHK(upload(&gr.ids_d, kv.second.ids));
+      HIPCHK(upload(&gr.lo_d, kv.second.lo));
+    }
+  }
+  std::vector<uint32_t> nm(b->nblk);
+  std::vector<int> part;
+  for (int i = 0; i < b->nblk; i++) {
+    nm[i] = b->amr_remap_blk[i] == 0 ? 0u : all_sectors & ~b->amr_local[i];
+    if (b->amr_remap_blk[i] == 2) part.push_back(i);
+  }
+  HIPCHK(hipMalloc((void**)&b->amr_nmask_d, sizeof(uint32_t) * nm.size()));
+  HIPCHK(hipMemcpy(b->amr_nmask_d, nm.data(), sizeof(uint32_t) * nm.size(), hipMemcpyHostToDevice));
+  HIPCHK(upload(&b->partial_ids_d, part));
   return SPARK_OK;
 }
 
@@ -1570,7 +1736,7 @@ int spark_set_amr_grid(spark_batch* b, int nbx0, int nby0, int nbz0, const int* 
   b->amr_local.assign(b->nblk, 0);
   b->amr_remap_count = 0;
   b->amr_partial_count = 0;
-  if (b->fused && n >= b->p.nguard) {
+  if (n >= b->p.nguard) {
     std::vector<int64_t> nb((size_t)b->nblk * 27, -1);
     const uint32_t all_sectors = ((1u << 27) - 1) & ~(1u << 13);
     for (int i = 0; i < b->nblk; i++) {
@@ -1636,6 +1802,10 @@ int spark_set_amr_grid(spark_batch* b, int nbx0, int nby0, int nbz0, const int* 
       HIPCHK(hipMemcpy(b->amr_smask_d, sm.data(), sizeof(uint32_t) * sm.size(), hipMemcpyHostToDevice));
     }
     b->planned = false;
+  }
+  if (!b->fused) {
+    int rc = plain_groups_build(b);
+    if (rc) return rc;
   }
   // faces with a finer leaf across (the region across a face is one block
   // position of the block's level: one leaf, or finer leaves only)

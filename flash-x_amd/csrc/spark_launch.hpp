@@ -46,6 +46,10 @@ struct PlainLaunch {
   const int* blist;       // device list of block ids in this shape class
   int nblk;               // length of blist
   int nx, ny, nz;         // interior shape of the class
+  // stage regions other than interior + ngoff: ext cells from blo[3 q ..] of
+  // entry q of blist (blo nullptr: the interior grown by ngoff)
+  const int* blo;
+  int ext[3];
   const double* U0;       // step input (hy_tmpState role); also holds SHOK
   const double* Sin;      // stage input state (U at stage 1, S after)
   double* Sout;           // stage output state (U at the last stage, S before)

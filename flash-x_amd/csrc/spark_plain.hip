@@ -50,6 +50,21 @@ __device__ __forceinline__ Lims stage_lims(const DevParams& P, const BlockMeta& 
   return L;
 }
 
+// region of a stage launch's entry q: the interior grown by ngoff, or with blo
+// the box of `ext` cells that starts there
+struct Ext { int n[3]; };
+__device__ __forceinline__ Lims entry_lims(const DevParams& P, const BlockMeta& m, int ngoff, const int* __restrict__ blo,
+                                           const Ext& ext, int q) {
+  if (blo == nullptr) return stage_lims(P, m, ngoff);
+  Lims L;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    L.lo[d] = blo[3 * q + d];
+    L.hi[d] = L.lo[d] + ext.n[d] - 1;
+  }
+  return L;
+}
+
 __device__ __forceinline__ int64_t cix(const BlockMeta& m, int i, int j, int k) {
   return (int64_t)i + (int64_t)m.NX * ((int64_t)j + (int64_t)m.NY * (int64_t)k);
 }
@@ -64,11 +79,12 @@ __device__ __forceinline__ int64_t fix(const BlockMeta& m, int i, int j, int k) 
 template <int NDIM>
 __global__ void __launch_bounds__(256) k_flatten(DevParams P, const BlockMeta* __restrict__ meta,
                                                  const int* __restrict__ blist, const double* __restrict__ S,
-                                                 double* __restrict__ flat, int ngoff) {
+                                                 double* __restrict__ flat, int ngoff, const int* __restrict__ blo,
+                                                 Ext ext) {
   int cx, cy;
   xcd_chunk(cx, cy);
   const BlockMeta m = meta[blist[cy]];
-  Lims L = stage_lims(P, m, ngoff);
+  Lims L = entry_lims(P, m, ngoff, blo, ext, cy);
   const int kx = 1, ky = (NDIM > 1), kz = (NDIM == 3);
   const int lo0 = L.lo[0] - kx, lo1 = L.lo[1] - ky, lo2 = L.lo[2] - kz;
   const int ex = L.hi[0] + kx - lo0 + 1, ey = L.hi[1] + ky - lo1 + 1, ez = L.hi[2] + kz - lo2 + 1;
@@ -253,7 +269,8 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
                                                const int* __restrict__ blist, const double* __restrict__ S,
                                                const double* __restrict__ Ushok, const double* __restrict__ flat,
                                                int ngoff, int lanes, int* __restrict__ err,
-                                               double* __restrict__ fb, double weight, int add, UpdArgs UA) {
+                                               double* __restrict__ fb, double weight, int add, UpdArgs UA,
+                                               const int* __restrict__ blo, Ext ext) {
   constexpr int R = ReconRadius<RECON>::R;
   constexpr int NFM = F_NUM + NSM;
   extern __shared__ double sm[];
@@ -261,7 +278,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
   int bx, by;
   xcd_chunk(bx, by);
   const BlockMeta m = meta[blist[by]];
-  Lims L = stage_lims(P, m, ngoff);
+  Lims L = entry_lims(P, m, ngoff, blo, ext, by);
   constexpr int T1 = (DIR == 0) ? 1 : 0;
   constexpr int T2 = (DIR == 2) ? 1 : 2;
   const int Lr = L.hi[DIR] - L.lo[DIR] + 3;
@@ -999,18 +1016,20 @@ static int resident_waves(const void* kern, int threads, size_t shm) {
   return res;
 }
 
+static Ext region_ext(const PlainLaunch& L, int ngoff) {
+  const int n[3] = {L.nx, L.ny, L.nz};
+  Ext E;
+  for (int d = 0; d < 3; d++) E.n[d] = L.blo ? L.ext[d] : d < L.P.ndim ? n[d] + 2 * ngoff : 1;
+  return E;
+}
+
 template <int DIR, int RECON, int RIEMANN, int NSM, int STEP>
 static hipError_t launch_flux_t(const PlainLaunch& L, int ngoff, const UpdArgs& UA) {
-  // geometry of this stage (all blocks in the list share one shape)
-  const int n[3] = {L.nx, L.ny, L.nz};
-  int lo[3], hi[3];
-  for (int d = 0; d < 3; d++) {
-    if (d < L.P.ndim) { lo[d] = L.P.ng - ngoff; hi[d] = L.P.ng + n[d] - 1 + ngoff; }
-    else { lo[d] = 0; hi[d] = 0; }
-  }
+  // region of this stage (all entries of the list share one shape)
+  const Ext E = region_ext(L, ngoff);
   const int T1 = (DIR == 0) ? 1 : 0, T2 = (DIR == 2) ? 1 : 2;
-  const int Lr = hi[DIR] - lo[DIR] + 3;
-  const int nt1 = hi[T1] - lo[T1] + 1, nt2 = hi[T2] - lo[T2] + 1;
+  const int Lr = E.n[DIR] + 2;
+  const int nt1 = E.n[T1], nt2 = E.n[T2];
   // LDS slots per thread: the hydro face states, 5 centred values and the
   // shock flag; then the scalars' face states; then the face fluxes
   constexpr int LDSV = (R_NUM + 6 > F_NUM + NSM) ? R_NUM + 6 : F_NUM + NSM;
@@ -1081,7 +1100,7 @@ static hipError_t launch_flux_t(const PlainLaunch& L, int ngoff, const UpdArgs& 
     L.prof->begin(L.stream, names[DIR], bytes, flops);
   }
   hipLaunchKernelGGL((k_flux<DIR, RECON, RIEMANN, NSM, STEP>), grid, block, shm, L.stream, L.P, L.meta, L.blist,
-                     L.Sin, L.U0, L.flat, ngoff, lanes, L.err, L.fb[DIR], L.weight, L.add_flux, UA);
+                     L.Sin, L.U0, L.flat, ngoff, lanes, L.err, L.fb[DIR], L.weight, L.add_flux, UA, L.blo, E);
   if (L.prof) L.prof->end(L.stream);
   return hipGetLastError();
 }
@@ -1107,23 +1126,20 @@ static hipError_t launch_flux_r(const PlainLaunch& L, int ngoff, const UpdArgs& 
 
 hipError_t plain_stage(const PlainLaunch& L, int ngoff, double c1, double c2, double c3, int final_stage) {
   hipError_t e;
-  const int n[3] = {L.nx, L.ny, L.nz};
-  int boxf = 1;
-  for (int d = 0; d < L.P.ndim; d++) boxf *= n[d] + 2 * ngoff + 2;
+  const Ext E = region_ext(L, ngoff);
   if (L.P.use_flat && L.P.recon == RECON_WENO5) {
-    if (L.prof) {
-      int bx = 1, bxr = 1;
-      for (int d = 0; d < L.P.ndim; d++) { bx *= n[d] + 2 * ngoff + 2; bxr *= n[d] + 2 * ngoff + 6; }
+    int bx = 1, bxr = 1;
+    for (int d = 0; d < L.P.ndim; d++) { bx *= E.n[d] + 2; bxr *= E.n[d] + 6; }
+    if (L.prof)
       L.prof->begin(L.stream, "k_flatten", 8.0 * L.nblk * ((double)bxr * (2 + L.P.ndim) + bx),
                     (double)L.nblk * bx * 25.0 * L.P.ndim);
-    }
-    const dim3 fg(grid_x_for(boxf, 512), L.nblk), fb(256);
+    const dim3 fg(grid_x_for(bx, 512), L.nblk), fb(256);
     if (L.P.ndim == 3)
-      hipLaunchKernelGGL(k_flatten<3>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff);
+      hipLaunchKernelGGL(k_flatten<3>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff, L.blo, E);
     else if (L.P.ndim == 2)
-      hipLaunchKernelGGL(k_flatten<2>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff);
+      hipLaunchKernelGGL(k_flatten<2>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff, L.blo, E);
     else
-      hipLaunchKernelGGL(k_flatten<1>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff);
+      hipLaunchKernelGGL(k_flatten<1>, fg, fb, 0, L.stream, L.P, L.meta, L.blist, L.Sin, L.flat, ngoff, L.blo, E);
     if (L.prof) L.prof->end(L.stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }

@@ -1,4 +1,4 @@
-// spark_regions.hpp -- stage regions of the batched forms as boxes of a
+// spark_regions.hpp -- stage regions on a block hierarchy as boxes of a
 // block's guard-celled index space (host code), and the boundary cells of a
 // box (host and device).
 #pragma once
@@ -115,6 +115,41 @@ inline void sector_boxes(int nx, int ny, int nz, int g, int e, uint32_t local, s
     }
   }
   flush(prev);
+}
+
+// The computed sectors alone, without the interior, as disjoint boxes: the
+// largest union of sectors that is a box first (in sectors; 0 and +-1 per
+// dimension have at most 6 ranges), until none is left.  The plain form's
+// sweeps run every block's interior in one launch and these boxes in one
+// launch per box shape, so few large boxes count; a level change across one
+// face gives one slab.
+inline void outer_boxes(int nx, int ny, int nz, int g, int e, uint32_t local, std::vector<Box>& out) {
+  if (e <= 0) return;
+  const int n[3] = {nx, ny, nz};
+  uint32_t left = local & ((1u << 27) - 1) & ~(1u << 13);
+  while (left) {
+    int best = 0, lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+    uint32_t take = 0;
+    for (int r = 0; r < 216; r++) {
+      static const int ra[6] = {-1, 0, 1, -1, 0, -1}, rb[6] = {-1, 0, 1, 0, 1, 1};
+      const int q[3] = {r % 6, r / 6 % 6, r / 36};
+      uint32_t m = 0;
+      for (int oz = ra[q[2]]; oz <= rb[q[2]]; oz++)
+        for (int oy = ra[q[1]]; oy <= rb[q[1]]; oy++)
+          for (int ox = ra[q[0]]; ox <= rb[q[0]]; ox++) m |= 1u << (13 + ox + 3 * oy + 9 * oz);
+      int cells = 1;
+      for (int d = 0; d < 3; d++) cells *= (ra[q[d]] < 0 ? e : 0) + (ra[q[d]] <= 0 && rb[q[d]] >= 0 ? n[d] : 0) + (rb[q[d]] > 0 ? e : 0);
+      if ((m & left) != m || cells <= best) continue;
+      best = cells;
+      take = m;
+      for (int d = 0; d < 3; d++) {
+        lo[d] = ra[q[d]] < 0 ? g - e : ra[q[d]] == 0 ? g : g + n[d];
+        hi[d] = rb[q[d]] < 0 ? g - 1 : rb[q[d]] == 0 ? g + n[d] - 1 : g + n[d] + e - 1;
+      }
+    }
+    out.push_back(Box{lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]});
+    left &= ~take;
+  }
 }
 
 }  // namespace spark

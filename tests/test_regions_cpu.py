@@ -37,3 +37,15 @@ def test_boundary_cells_visit_each_boundary_cell_once(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     print(r.stdout.strip())
     assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
+def test_outer_boxes_cover_the_computed_sectors_exactly(tmp_path):
+    """The plain form's boxes beside the interior (spark_regions.hpp), over
+    the same masks and depths."""
+    exe = tmp_path / "check_outer_boxes"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", str(ROOT / "flash-x_amd" / "csrc"),
+                    str(ROOT / "tests" / "cpp" / "check_outer_boxes.cpp"), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    print(r.stdout.strip())
+    assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout
