@@ -123,9 +123,7 @@ struct spark_batch {
   int amr_remap_count = 0;
   int amr_partial_count = 0;
   // plain form on a block hierarchy: per stage the boxes its sweeps run, one
-  // group per box shape (plain_groups_build); the guard sectors a block takes
-  // from same-level leaves between the stages, and the blocks with some but
-  // not all of them
+  // group per box shape (plain_groups_build)
   struct PlainGroup {
     int ext[3];
     int n;
@@ -134,8 +132,6 @@ struct spark_batch {
     int* lo_d;
   };
   std::vector<PlainGroup> groups[3];
-  uint32_t* amr_nmask_d = nullptr;
-  int* partial_ids_d = nullptr;
   bool same_level = true;      // SPARK_OPT_SAME_LEVEL_HALOS
   int* remap_ids_d = nullptr;  // the remapping blocks
   int* tele_ids_d = nullptr;   // the telescoping blocks
@@ -210,6 +206,7 @@ PlainLaunch make_launch(spark_batch* b, const ShapeClass& c) {
   L.nblk = (int)c.ids.size();
   L.nx = c.nx; L.ny = c.ny; L.nz = c.nz;
   L.blo = nullptr;
+  L.nbr = nullptr;
   L.ext[0] = L.ext[1] = L.ext[2] = 0;
   L.U0 = b->U;
   L.Sin = b->S;
@@ -236,20 +233,15 @@ int required_guard(const spark_params& p) {
   return maxoff + (fused ? std::max(p.nstencil, 3) : p.nstencil);
 }
 
-bool fused_remap(const spark_batch* b);
+bool ug_remap(const spark_batch* b);
 void drop_graph(spark_batch* b);
 
-// batched forms on a block hierarchy: same-level halos in use
+// block hierarchy: same-level halos in use.  The guard sectors across which
+// lies a leaf of the block's own level are read from that leaf, and a block
+// computes only its interior and the other sectors.  The values are those of
+// telescoping (the same cells from the same inputs).
 bool amr_remap_on(const spark_batch* b) {
-  return b->fused && b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
-}
-
-// plain form on a block hierarchy: the guard sectors across which lies a leaf
-// of the block's own level are copied from that leaf between the stages, and
-// a block computes only its interior and the other sectors.  The values are
-// those of telescoping (the same cells from the same inputs).
-bool plain_same_level(const spark_batch* b) {
-  return b->amr && !b->fused && b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
+  return b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
 }
 
 void free_plain_groups(spark_batch* b) {
@@ -260,10 +252,6 @@ void free_plain_groups(spark_batch* b) {
     }
     st.clear();
   }
-  if (b->amr_nmask_d) (void)hipFree(b->amr_nmask_d);
-  if (b->partial_ids_d) (void)hipFree(b->partial_ids_d);
-  b->amr_nmask_d = nullptr;
-  b->partial_ids_d = nullptr;
 }
 
 int run_dt(spark_batch* b, int hist_slot) {
@@ -278,10 +266,6 @@ int run_dt(spark_batch* b, int hist_slot) {
                                hist_slot >= 0 && b->dt_control ? b->dtctl_d : nullptr));
   return SPARK_OK;
 }
-
-// layers around the interior that a stage of it and the step's shock
-// detection (hybrid solver: of the layer around it too) read
-int interior_reach(const spark_batch* b) { return std::max(b->p.nstencil, b->p.use_hybrid_riemann ? 2 : 1); }
 
 // Guard fill of a uniform block grid.  full: every variable over every
 // guard layer (Grid_fillGuardCells semantics).  Otherwise only what the
@@ -315,19 +299,6 @@ int run_fill(spark_batch* b, double* pool, bool full, int depth) {
       L.blist = b->tele_ids_d;
       L.nblk = b->n_tele;
       HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth, b->p.use_hybrid_riemann ? nullptr : b->amr_smask_d, 1));
-    }
-  } else if (b->amr && !full && plain_same_level(b)) {
-    // blocks with same-level leaves all around: the layers stage 1 of the
-    // interior reads; the others to the depth they telescope from
-    if (b->amr_remap_count > 0) {
-      L.blist = b->remap_ids_d;
-      L.nblk = b->amr_remap_count;
-      HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, interior_reach(b)));
-    }
-    if (b->n_tele > 0) {
-      L.blist = b->tele_ids_d;
-      L.nblk = b->n_tele;
-      HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth));
     }
   } else if (b->amr) {
     HIPCHK(spark::amr_fill(L, b->amr_g, pool, vl, depth));
@@ -385,12 +356,11 @@ int run_amr_correct(spark_batch* b) {
 
 // first-stage guard reach: stencil extent of stage 1 beyond the interior
 int stage1_reach(const spark_batch* b) {
-  // the remapping batched forms only need the layers shockDetect reads: one
-  // for the interior, two when the hybrid solver reads SHOK one layer out
-  if (fused_remap(b)) return b->p.use_hybrid_riemann ? 2 : 1;
   return (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + b->p.nstencil;
 }
 
+// same_level: the stages that follow may read same-level halos (a whole step;
+// the plain form's stage entry points telescope over the block's own guards)
 int run_step_begin(spark_batch* b, bool same_level = false) {
   // SHOK over the cells the stages' hybrid Riemann solves read: the stage-1
   // region plus one layer (the reference computes NGUARD-1 layers; the
@@ -402,19 +372,7 @@ int run_step_begin(spark_batch* b, bool same_level = false) {
   // own in the stages) get it one layer out.
   const bool hyb = b->p.use_hybrid_riemann != 0;
   const int band = !hyb ? 0 : (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + 1;
-  if (same_level && plain_same_level(b)) {
-    PlainLaunch L = make_launch(b, b->classes[0]);
-    if (b->n_tele > 0) {
-      L.blist = b->tele_ids_d;
-      L.nblk = b->n_tele;
-      HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, band));
-    }
-    if (b->amr_remap_count > 0) {
-      L.blist = b->remap_ids_d;
-      L.nblk = b->amr_remap_count;
-      HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, hyb ? 1 : 0));
-    }
-  } else if (amr_remap_on(b)) {
+  if (amr_remap_on(b) && (b->fused || same_level)) {
     // a hierarchy has one block shape
     PlainLaunch L = make_launch(b, b->classes[0]);
     if (b->n_tele > 0) {
@@ -427,6 +385,9 @@ int run_step_begin(spark_batch* b, bool same_level = false) {
       L.nblk = b->amr_remap_count;
       HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, hyb ? 1 : 0, b->nbr_d));
     }
+  } else if (same_level && ug_remap(b)) {
+    PlainLaunch L = make_launch(b, b->classes[0]);
+    HIPCHK(spark::plain_shock_detect(L, b->U, b->flat, band, b->nbr_d));
   } else {
     for (auto& c : b->classes) {
       PlainLaunch L = make_launch(b, c);
@@ -486,10 +447,13 @@ hipError_t fused_launch(const spark_batch* b, const spark::FusedArgs& A, int gri
   return b->fused64 ? spark::fused_stage_f64(A, grid, lds, g_stream) : spark::fused_stage_f32(A, grid, lds, g_stream);
 }
 
-// the batched forms on a uniform grid in refill mode read halo cells from
-// the neighbouring blocks, so no guard fill runs between stages
-bool fused_remap(const spark_batch* b) {
-  return b->fused && b->has_ug && b->p.guard_mode == SPARK_GUARD_REFILL;
+// 3D blocks of a uniform grid in refill mode read halo cells from the
+// neighbouring blocks (each at least as wide as a stencil reaches), so a step
+// fills no guard cells: on 64 blocks of 16^3 the three fills of a plain step
+// took 0.083 of 0.43 ms
+bool ug_remap(const spark_batch* b) {
+  const BlockMeta& m = b->meta_h[0];
+  return b->has_ug && b->p.guard_mode == SPARK_GUARD_REFILL && b->p.ndim == 3 && std::min({m.nx, m.ny, m.nz}) >= 3;
 }
 
 spark::FusedArgs fused_args(spark_batch* b, int stage) {
@@ -505,7 +469,7 @@ spark::FusedArgs fused_args(spark_batch* b, int stage) {
   A.Sin = stage_in(b, stage);
   A.Sout = stage_out(b, stage);
   for (int d = 0; d < 3; d++) A.fb[d] = b->p.flux_correct ? b->fb[d] : nullptr;
-  A.nbr = (fused_remap(b) || amr_remap_on(b)) ? b->nbr_d : nullptr;
+  A.nbr = (ug_remap(b) || amr_remap_on(b)) ? b->nbr_d : nullptr;
   A.weight = b->weights[stage - 1];
   A.add_flux = stage > 1;
   A.dtp = b->dtp;
@@ -520,7 +484,7 @@ spark::FusedArgs fused_args(spark_batch* b, int stage) {
 // saveState's copy is folded away: stage 1 reads the solution U directly
 // (hy_starState == Uin at stage 1) and the last stage writes U directly
 // (updateState copies exactly the last stage's region, the interior).
-int run_stage(spark_batch* b, int stage, int ngoff) {
+int run_stage(spark_batch* b, int stage, int ngoff, bool same_level = false) {
   const double* co = b->coeff[stage - 1];
   if (stage != b->last_stage) b->star = stage_out(b, stage);
   if (b->fused) {
@@ -546,13 +510,13 @@ int run_stage(spark_batch* b, int stage, int ngoff) {
     L.add_flux = stage > 1;
     L.Sin = stage_in(b, stage);
     L.Sout = stage_out(b, stage);
+    if (same_level && ug_remap(b)) L.nbr = b->nbr_d;
     HIPCHK(spark::plain_stage(L, ngoff, co[0], co[1], co[2], stage == b->last_stage));
   }
   return SPARK_OK;
 }
 
-// one stage of the plain form over the boxes of its groups, then the guard
-// sectors the next stage reads from same-level leaves, copied from them
+// one stage of the plain form on a hierarchy over the boxes of its groups
 int run_stage_groups(spark_batch* b, int stage) {
   const double* co = b->coeff[stage - 1];
   double* out = stage_out(b, stage);
@@ -566,28 +530,13 @@ int run_stage_groups(spark_batch* b, int stage) {
     PlainLaunch G = L;
     G.blist = g.ids_d;
     G.blo = g.lo_d;
+    G.nbr = b->nbr_d;
     G.nblk = g.n;
     for (int d = 0; d < 3; d++) {
       G.ext[d] = g.ext[d];
       if (!g.interior) G.fb[d] = nullptr;
     }
     HIPCHK(spark::plain_stage(G, 0, co[0], co[1], co[2], stage == b->last_stage));
-  }
-  if (stage == b->last_stage) return SPARK_OK;
-  spark::VarList vl;
-  vl.n = 0;
-  const int need[7] = {spark::V_DENS, spark::V_EINT, spark::V_GAMC, spark::V_PRES, spark::V_VELX, spark::V_VELY, spark::V_VELZ};
-  for (int v : need) vl.v[vl.n++] = v;
-  for (int s = 0; s < b->p.nscalars; s++) vl.v[vl.n++] = spark::V_NPROP + s;
-  if (b->amr_remap_count > 0) {
-    L.blist = b->remap_ids_d;
-    L.nblk = b->amr_remap_count;
-    HIPCHK(spark::amr_fill(L, b->amr_g, out, vl, b->p.nstencil));
-  }
-  if (b->amr_partial_count > 0) {
-    L.blist = b->partial_ids_d;
-    L.nblk = b->amr_partial_count;
-    HIPCHK(spark::amr_fill(L, b->amr_g, out, vl, b->limits_array[stage] + b->p.nstencil, b->amr_nmask_d, 0));
   }
   return SPARK_OK;
 }
@@ -600,15 +549,15 @@ int run_step_end(spark_batch* b) {
 int run_full_step(spark_batch* b) {
   int rc;
   if ((rc = run_step_begin(b, true))) return rc;
-  if (plain_same_level(b)) {
+  if (!b->fused && amr_remap_on(b)) {
     for (int s = 1; s <= b->last_stage; s++)
       if ((rc = run_stage_groups(b, s))) return rc;
     return run_step_end(b);
   }
   const bool refill = b->p.guard_mode == SPARK_GUARD_REFILL;
   for (int s = 1; s <= b->last_stage; s++) {
-    if ((rc = run_stage(b, s, refill ? 0 : b->limits_array[s - 1]))) return rc;
-    if (refill && s < b->last_stage && !fused_remap(b))
+    if ((rc = run_stage(b, s, refill ? 0 : b->limits_array[s - 1], true))) return rc;
+    if (refill && s < b->last_stage && !ug_remap(b))
       if ((rc = run_fill(b, stage_out(b, s), false, b->p.nstencil))) return rc;
   }
   return run_step_end(b);
@@ -878,7 +827,6 @@ int fused_plan(spark_batch* b) {
 int plain_groups_build(spark_batch* b) {
   free_plain_groups(b);
   const int g = b->p.nguard;
-  const uint32_t all_sectors = ((1u << 27) - 1) & ~(1u << 13);
   auto upload = [](int** dst, const std::vector<int>& v) -> hipError_t {
     hipError_t e = hipMalloc((void**)dst, sizeof(int) * std::max<size_t>(1, v.size()));
     return e == hipSuccess ? hipMemcpy(*dst, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice) : e;
@@ -911,15 +859,6 @@ int plain_groups_build(spark_batch* b) {
       HIPCHK(upload(&gr.lo_d, kv.second.lo));
     }
   }
-  std::vector<uint32_t> nm(b->nblk);
-  std::vector<int> part;
-  for (int i = 0; i < b->nblk; i++) {
-    nm[i] = b->amr_remap_blk[i] == 0 ? 0u : all_sectors & ~b->amr_local[i];
-    if (b->amr_remap_blk[i] == 2) part.push_back(i);
-  }
-  HIPCHK(hipMalloc((void**)&b->amr_nmask_d, sizeof(uint32_t) * nm.size()));
-  HIPCHK(hipMemcpy(b->amr_nmask_d, nm.data(), sizeof(uint32_t) * nm.size(), hipMemcpyHostToDevice));
-  HIPCHK(upload(&b->partial_ids_d, part));
   return SPARK_OK;
 }
 
@@ -1371,7 +1310,7 @@ int spark_hydro_step(spark_batch* b, double dt, double dtOld) {
     return fail(SPARK_ERR_STATE, "refill guard mode needs spark_set_uniform_grid");
   HIPCHK(spark::plain_set_scalar(g_stream, b->dtp, dt));
   int rc;
-  if ((b->has_ug || b->amr) && (rc = run_fill(b, b->U, false, stage1_reach(b)))) return rc;
+  if ((b->has_ug || b->amr) && !ug_remap(b) && (rc = run_fill(b, b->U, false, stage1_reach(b)))) return rc;
   if ((rc = run_full_step(b))) return rc;
   if (b->amr && b->p.flux_correct) return run_amr_correct(b);
   return SPARK_OK;
@@ -1401,7 +1340,7 @@ int spark_step_end(spark_batch* b) {
 static int one_step(spark_batch* b) {
   int rc = run_dt(b, 0);
   if (rc) return rc;
-  if ((b->has_ug || b->amr) && (rc = run_fill(b, b->U, false, stage1_reach(b)))) return rc;
+  if ((b->has_ug || b->amr) && !ug_remap(b) && (rc = run_fill(b, b->U, false, stage1_reach(b)))) return rc;
   if ((rc = run_full_step(b))) return rc;
   if (b->amr && b->p.flux_correct) return run_amr_correct(b);
   return SPARK_OK;

@@ -50,6 +50,9 @@ struct PlainLaunch {
   // entry q of blist (blo nullptr: the interior grown by ngoff)
   const int* blo;
   int ext[3];
+  // 3D, optional: per block 27 pool offsets of the blocks around it; guard
+  // cells of the stage input are then read from those blocks (cell_at)
+  const int64_t* nbr;
   const double* U0;       // step input (hy_tmpState role); also holds SHOK
   const double* Sin;      // stage input state (U at stage 1, S after)
   double* Sout;           // stage output state (U at the last stage, S before)

@@ -408,3 +408,26 @@ def test_graph_replays_match_eager_steps_on_the_hierarchy(form):
         assert np.array_equal(de, dg), s
         nd = sum(int(np.count_nonzero(x != y)) for x, y in zip(interiors(prob, oe), interiors(prob, og)))
         assert nd == 0, f"replay {s}: {nd} differing interior values"
+
+
+@pytest.mark.parametrize("recon,riemann,rk,nst,hybrid,nscalars", [
+    ("weno5", "hllc", 3, 3, 0, 3),
+    ("weno5", "hllc", 3, 3, 1, 0),
+    ("weno5", "hll", 2, 3, 0, 0),
+    ("mp5", "hllc", 2, 3, 1, 8),
+    ("plm", "hllc", 3, 2, 1, 1),
+    ("fog", "hll", 2, 1, 0, 0),
+])
+def test_plain_same_level_halos_equal_telescoping(recon, riemann, rk, nst, hybrid, nscalars):
+    """The plain form's sweeps and flattening through the neighbour table, over
+    interiors and the boxes beside them, agree bit for bit with telescoping
+    over every guard cell."""
+    prob = three_level(nscalars=nscalars, recon=recon, riemann=riemann, rk_order=rk, nstencil=nst,
+                       **(SHOCKED if hybrid else {}))
+    full, some = same_level_blocks(prob)
+    assert full > 0 and some > 0
+    d_on, o_on, _ = run(prob, 2, "plain_fp64")
+    d_off, o_off, _ = run(prob, 2, "plain_fp64", same_level_halos=0)
+    assert np.array_equal(d_on, d_off)
+    for x, y in zip(interiors(prob, o_on), interiors(prob, o_off)):
+        assert np.array_equal(x, y)

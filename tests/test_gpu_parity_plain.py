@@ -431,3 +431,35 @@ def test_geometry_is_refused_where_it_is_not_implemented():
             b.set_geometry("spherical", rows)
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("nb,n,kw", [
+    ((2, 2, 2), (16, 16, 16), {}),
+    ((3, 1, 2), (3, 5, 4), {}),
+    ((1, 2, 3), (7, 16, 3), dict(recon="mp5", use_hybrid_riemann=1)),
+    ((2, 3, 1), (33, 4, 9), dict(recon="plm", nstencil=2, rk_order=2, nscalars=2)),
+    ((2, 1, 2), (5, 6, 17), dict(recon="fog", nstencil=1, riemann="hll", use_hybrid_riemann=1)),
+    ((3, 2, 2), (2, 4, 4), {}),  # narrower than a stencil reaches: filled guards
+])
+def test_refill_3d_block_shapes(nb, n, kw):
+    """Refill mode of 3D blocks, where every stage reads its halos from the
+    neighbouring blocks (outflow at the domain faces)."""
+    cfg = problems.base_cfg(ndim=3, nguard=6, guard_mode="refill", cfl=0.3, **kw)
+    r = np.random.default_rng(3)
+    dx = 1.0 / 32
+    blocks, arrays = [], []
+    for bk in range(nb[2]):
+        for bj in range(nb[1]):
+            for bi in range(nb[0]):
+                b = dict(nx=n[0], ny=n[1], nz=n[2], level=1, dx=dx, dy=dx, dz=dx)
+                NZ, NY, NX = problems.gc_shape(cfg, b)
+                Z, Y, X = problems._centers(cfg, b, (bi * n[0] * dx, bj * n[1] * dx, bk * n[2] * dx), NZ, NY, NX)
+                s = np.sin(7 * X + 3 * Y) * np.cos(5 * Z - 2 * Y)
+                U = np.zeros((NZ, NY, NX, capi.SPARK_NPROP + cfg["nscalars"]))
+                scal = [0.5 + 0.4 * np.sin((q + 2) * X + Z) for q in range(cfg["nscalars"])]
+                problems.fill_thermo(U, 1.0 + 0.5 * s, np.where(X + Y + Z < 0.6, 5.0, 1.0) + 0.1 * s, 0.3 * s, -0.2 * s, 0.1 * s,
+                                     1.4, scalars=scal)
+                U[:] *= 1.0 + 1e-3 * r.random(U.shape[:-1])[..., None]
+                blocks.append(b)
+                arrays.append(U)
+    run_case(problems.Problem("refill", cfg, blocks, arrays, ug=nb), 3, f"refill {nb} x {n}")
