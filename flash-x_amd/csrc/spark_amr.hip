@@ -14,8 +14,8 @@
 namespace spark {
 namespace {
 
-__device__ __forceinline__ int64_t acix(int NX, int i, int j, int k) {
-  return (int64_t)i + (int64_t)NX * ((int64_t)j + (int64_t)NX * (int64_t)k);
+__device__ __forceinline__ int64_t acix(int PX, int NX, int i, int j, int k) {
+  return (int64_t)i + (int64_t)PX * ((int64_t)j + (int64_t)NX * (int64_t)k);
 }
 
 __device__ __forceinline__ int leaf_at(const AmrGrid& G, int L, const int gi[3]) {
@@ -86,7 +86,7 @@ __device__ __forceinline__ Src amr_src(const BlockMeta* __restrict__ meta, const
   }
   Src r;
   r.avg = !coarse;
-  r.off = ms.base + acix(NX, c[0], c[1], c[2]);
+  r.off = ms.base + acix(ms.PX, NX, c[0], c[1], c[2]);
   return r;
 }
 
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) k_amr_fill(DevParams P, const BlockMeta* 
   const int ext = n + 2 * depth;
   const int total = ext * ext * ext;
   const int o[3] = {G.org[3 * bid], G.org[3 * bid + 1], G.org[3 * bid + 2]};
-  const Shape S{m.NX, (int64_t)m.NX * m.NX, m.cstride};
+  const Shape S{m.PX, (int64_t)m.PX * m.NX, m.cstride};
   const uint32_t mk = smask ? smask[bid] : ~0u;
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
     const int loc[3] = {g - depth + t % ext, g - depth + (t / ext) % ext, g - depth + t / (ext * ext)};
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(256) k_amr_fill(DevParams P, const BlockMeta* 
     if (inside) continue;
     if (dep > keep && !((mk >> sec) & 1u)) continue;
     const int flip = amr_domain(G, L, gi);
-    const int64_t dst = m.base + acix(m.NX, loc[0], loc[1], loc[2]);
+    const int64_t dst = m.base + acix(m.PX, m.NX, loc[0], loc[1], loc[2]);
     const int s = leaf_at(G, L, gi);
     if (meta[s].level != L - 1) {
       // copy / restriction: the loads of a chunk of variables are issued

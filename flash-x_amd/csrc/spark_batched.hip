@@ -260,7 +260,7 @@ __device__ __forceinline__ void xy_face(const FusedArgs& A, const BlockMeta& m, 
   bool shk = false;
   if (RIEMANN == RIEMANN_HLLC_HYBRID) {
     const int64_t hi = bcix(m, I.x0 + fi, I.y0 + fj, k);
-    shk = face_in_shock(A.U0, m, hi - (DIR == 0 ? 1 : m.NX), hi);
+    shk = face_in_shock(A.U0, m, hi - (DIR == 0 ? 1 : m.PX), hi);
   }
   hydro_face<DIR, RIEMANN>(rp, Ls, Rs, cl, cr, F, A.err, shk);
 #pragma unroll
@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
     Real* mxb = lds + L.mx;
     Real* myb = lds + L.my;
     const int64_t cs = m.cstride;
-    const int64_t sz = (int64_t)m.NX * m.NY;
+    const int64_t sz = (int64_t)m.PX * m.NY;
     const double* sin = A.Sin + m.base;
     const double* S = A.Sin;  // pool base: cell_at() offsets include the block's base
     // the item's neighbour offsets, cached in LDS (read on every halo load)

@@ -26,7 +26,7 @@ struct FusedItem {
 constexpr int64_t NBR_EDGE = INT64_MIN;
 
 __device__ __forceinline__ int64_t bcix(const BlockMeta& m, int i, int j, int k) {
-  return (int64_t)i + (int64_t)m.NX * ((int64_t)j + (int64_t)m.NY * (int64_t)k);
+  return (int64_t)i + (int64_t)m.PX * ((int64_t)j + (int64_t)m.NY * (int64_t)k);
 }
 
 // pool offset of cell (i, j, k) of a block's guard-celled box.  With a
@@ -75,7 +75,7 @@ struct FusedArgs {
   // it: cells outside the block's interior are read from those neighbours
   // (uniform grid, guards not refilled between stages: NBR_EDGE where the
   // domain ends, outflow).  A sector the block computes itself (hierarchy:
-  // no leaf of its level across) holds base + ox nx + NX (oy ny + NY oz nz),
+  // no leaf of its level across) holds base + ox nx + PX (oy ny + NY oz nz),
   // which cell_at() turns into the block's own guard cell.  A row whose
   // centre entry is -1, or nullptr: the block reads its own guard cells.
   const int64_t* nbr;

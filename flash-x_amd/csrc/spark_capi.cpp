@@ -1018,6 +1018,15 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
 
   const int g = p->nguard;
   const int nf = 5 + p->nscalars;
+  // rows are padded (row_pad) unless that would take the state past half of a
+  // GPU's memory
+  int64_t padded = 0;
+  for (int i = 0; i < nblocks; i++) {
+    const int NX = blocks[i].nx + 2 * g;
+    padded += (int64_t)spark::row_pad(NX, g).pitch * (p->ndim > 1 ? blocks[i].ny + 2 * g : 1) *
+              (p->ndim > 2 ? blocks[i].nz + 2 * g : 1);
+  }
+  const bool pad_rows = padded * (3 * nvar + nf + 1) < (int64_t(128) << 30) / (int64_t)sizeof(double);
   std::map<std::tuple<int, int, int>, int> cls;
   int64_t max_int = 0;
   for (int i = 0; i < nblocks; i++) {
@@ -1034,12 +1043,14 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
     m.dx = bd.dx; m.dy = bd.dy; m.dz = bd.dz;
     m.level = bd.level; m.id = i;
     const int64_t ncell = (int64_t)m.NX * m.NY * m.NZ;
-    m.cstride = round_up(ncell, 64);
-    m.base = b->pool;
+    const spark::RowPad rp = pad_rows ? spark::row_pad(m.NX, g) : spark::RowPad{m.NX, 0};
+    m.PX = rp.pitch;
+    m.cstride = round_up(rp.lead + (int64_t)m.PX * m.NY * m.NZ, 64);
+    m.base = b->pool + rp.lead;
     b->pool += (int64_t)nvar * m.cstride;
-    m.obase = b->opool;
+    m.obase = b->opool + rp.lead;
     b->opool += m.cstride;
-    m.dbase = b->dpool;
+    m.dbase = b->dpool + rp.lead;
     b->dpool += (int64_t)nf * m.cstride;
     int64_t reg = 1;
     for (int q = 0; q < 3; q++) reg *= n[q] + (q < p->ndim ? 1 : 0);
@@ -1294,9 +1305,9 @@ int spark_compute_dt(spark_batch* b, double* dt, int minloc[5]) {
     const int bid = (int)loc[0];
     const BlockMeta& m = b->meta_h[bid < 0 || bid >= b->nblk ? 0 : bid];
     const long long c = loc[1];
-    minloc[0] = (int)(c % m.NX) + 1;
-    minloc[1] = (int)((c / m.NX) % m.NY) + 1;
-    minloc[2] = (int)(c / ((long long)m.NX * m.NY)) + 1;
+    minloc[0] = (int)(c % m.PX) + 1;
+    minloc[1] = (int)((c / m.PX) % m.NY) + 1;
+    minloc[2] = (int)(c / ((long long)m.PX * m.NY)) + 1;
     minloc[3] = m.level;
     minloc[4] = bid;
   }
@@ -1706,7 +1717,7 @@ int spark_set_amr_grid(spark_batch* b, int nbx0, int nby0, int nbz0, const int* 
               row[s] = b->meta_h[j].base;
             } else {
               // computed here: the entry cell_at() shifts back into this block
-              row[s] = mi.base + (int64_t)ox * mi.nx + (int64_t)mi.NX * ((int64_t)oy * mi.ny + (int64_t)mi.NY * oz * mi.nz);
+              row[s] = mi.base + (int64_t)ox * mi.nx + (int64_t)mi.PX * ((int64_t)oy * mi.ny + (int64_t)mi.NY * oz * mi.nz);
               local |= 1u << s;
             }
           }

@@ -497,6 +497,7 @@ struct BlockMeta {
   int64_t bbase;    // offset in the flux-register pools (interior faces)
   int nx, ny, nz;   // interior cells
   int NX, NY, NZ;   // guard-celled extents
+  int PX;           // doubles from one x row of the box to the next (row_pad: >= NX)
   double dx, dy, dz;
   int level, id;
 };

@@ -114,10 +114,7 @@ __device__ __forceinline__ void pencil_offsets(const BlockMeta& m, const int64_t
 }
 
 __device__ __forceinline__ int64_t cix(const BlockMeta& m, int i, int j, int k) {
-  return (int64_t)i + (int64_t)m.NX * ((int64_t)j + (int64_t)m.NY * (int64_t)k);
-}
-__device__ __forceinline__ int64_t fix(const BlockMeta& m, int i, int j, int k) {
-  return (int64_t)i + (int64_t)(m.NX + 1) * ((int64_t)j + (int64_t)(m.NY + 1) * (int64_t)k);
+  return (int64_t)i + (int64_t)m.PX * ((int64_t)j + (int64_t)m.NY * (int64_t)k);
 }
 
 // ---------------------------------------------------------------------------
@@ -138,7 +135,7 @@ __global__ void __launch_bounds__(256) k_flatten(DevParams P, const BlockMeta* _
   const int ex = L.hi[0] + kx - lo0 + 1, ey = L.hi[1] + ky - lo1 + 1, ez = L.hi[2] + kz - lo2 + 1;
   const int total = ex * ey * ez;
   const int64_t cs = m.cstride;
-  const int64_t str[3] = {1, (int64_t)m.NX, (int64_t)m.NX * m.NY};
+  const int64_t str[3] = {1, (int64_t)m.PX, (int64_t)m.PX * m.NY};
   const int velv[3] = {V_VELX, V_VELY, V_VELZ};
   const double betaMin = 0.75, betaMax = 0.85, Zmin = 0.25, Zmax = 0.75;
   __shared__ int64_t s_nb[NDIM == 3 ? 27 : 1];
@@ -365,7 +362,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
   ijk[T1] = L.lo[T1] + pen % nt1;
   ijk[T2] = L.lo[T2] + pen / nt1;
   const int64_t c = cix(m, ijk[0], ijk[1], ijk[2]);
-  const int64_t st = (DIR == 0) ? 1 : (DIR == 1) ? (int64_t)m.NX : (int64_t)m.NX * m.NY;
+  const int64_t st = (DIR == 0) ? 1 : (DIR == 1) ? (int64_t)m.PX : (int64_t)m.PX * m.NY;
   const double* sp = S + m.base;
   // pool offsets of the stencil's cells: in the block's own box, or through
   // the neighbour table
@@ -647,7 +644,7 @@ __global__ void __launch_bounds__(256) k_shock(DevParams P, const BlockMeta* __r
   const double* cp = vc + m.obase;
   const int64_t cs = m.cstride;
   const int ky = (P.ndim > 1), kz = (P.ndim == 3);
-  const int64_t sx = 1, sy = m.NX, sz = (int64_t)m.NX * m.NY;
+  const int64_t sx = 1, sy = m.PX, sz = (int64_t)m.PX * m.NY;
   const double beta = 0.5, delta = 0.1;
   for (int t = cx * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
     const int i = L.lo[0] + t % ex, j = L.lo[1] + (t / ex) % ey, k = L.lo[2] + t / (ex * ey);
@@ -1066,7 +1063,7 @@ __global__ void __launch_bounds__(256) k_aos_to_soa(const BlockMeta* __restrict_
   const int total = m.NX * m.NY * m.NZ;
   const double* src = aos + aos_off[blockIdx.y];
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x)
-    for (int v = 0; v < nvar; v++) U[m.base + v * m.cstride + t] = src[(int64_t)t * nunk + var_index[v]];
+    for (int v = 0; v < nvar; v++) U[m.base + v * m.cstride + box_cell(m, t)] = src[(int64_t)t * nunk + var_index[v]];
 }
 
 // ---------------------------------------------------------------------------

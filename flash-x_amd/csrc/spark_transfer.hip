@@ -21,11 +21,11 @@ namespace spark {
 namespace {
 
 __device__ __forceinline__ int64_t seg_cell(const BlockMeta& m, int ng, int ndim, int interior, int64_t t) {
-  if (!interior) return t;
+  if (!interior) return box_cell(m, t);
   const int i = (int)(t % m.nx);
   const int64_t row = t / m.nx;
   const int j = (int)(row % m.ny), k = (int)(row / m.ny);
-  return (ng + i) + (int64_t)m.NX * (j + (ndim > 1 ? ng : 0) + (int64_t)m.NY * (k + (ndim > 2 ? ng : 0)));
+  return (ng + i) + (int64_t)m.PX * (j + (ndim > 1 ? ng : 0) + (int64_t)m.NY * (k + (ndim > 2 ? ng : 0)));
 }
 
 // One thread per cell: the state side is coalesced; a wave's tuples are one
@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(256) k_unstage(const XferSeg* __restrict__ seg
   const BlockMeta m = meta[s.blk];
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < s.ncell; t += (int64_t)gridDim.x * blockDim.x) {
     const double* src = stage + (s.at + t) * width;
-    double* dst = pool + m.base + s.cell0 + t;
+    double* dst = pool + m.base + box_cell(m, s.cell0 + t);
     for (int v = 0; v < nvar; v++) dst[v * m.cstride] = src[slot[v]];
   }
 }

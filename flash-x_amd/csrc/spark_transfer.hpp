@@ -11,6 +11,7 @@
 #include <functional>
 #include <vector>
 
+#include "spark_launch.hpp"
 #include "spark_physics.hpp"
 
 namespace spark {
