@@ -1696,32 +1696,56 @@ int spark_set_amr_grid(spark_batch* b, int nbx0, int nby0, int nbz0, const int* 
       for (int d = 0; d < 3; d++) { bp[d] = origins[3 * i + d] / n; nbl[d] = nb0[d] << (L - 1); }
       int64_t row[27];
       uint32_t local = 0;
+      // the leaf of this block's level at block offset o, or -1
+      auto leaf = [&](const int (&o)[3]) -> int {
+        int q[3];
+        for (int d = 0; d < 3; d++) {
+          q[d] = bp[d] + o[d];
+          if (q[d] < 0 || q[d] >= nbl[d]) {
+            if (!per[d]) return -1;
+            q[d] = (q[d] + nbl[d]) % nbl[d];
+          }
+        }
+        const int j = map[((size_t)q[0] << sh) + (size_t)md[0] * (((size_t)q[1] << sh) + (size_t)md[1] * ((size_t)q[2] << sh))];
+        return b->meta_h[j].level == L ? j : -1;
+      };
+      // what cell_at() takes off a cell's offset in a sector's coordinates
+      auto shift = [&](const int (&o)[3]) -> int64_t {
+        return (int64_t)o[0] * mi.nx + (int64_t)mi.PX * ((int64_t)o[1] * mi.ny + (int64_t)mi.NY * o[2] * mi.nz);
+      };
+      bool any = false;
       for (int oz = -1; oz <= 1; oz++)
         for (int oy = -1; oy <= 1; oy++)
           for (int ox = -1; ox <= 1; ox++) {
             const int s = 13 + ox + 3 * oy + 9 * oz;
             if (s == 13) { row[s] = mi.base; continue; }
             const int o[3] = {ox, oy, oz};
-            int q[3];
-            bool in = true;
-            for (int d = 0; d < 3; d++) {
-              q[d] = bp[d] + o[d];
-              if (q[d] < 0 || q[d] >= nbl[d]) {
-                if (!per[d]) in = false;
-                q[d] = (q[d] + nbl[d]) % nbl[d];
-              }
-            }
-            int j = -1;
-            if (in) j = map[((size_t)q[0] << sh) + (size_t)md[0] * (((size_t)q[1] << sh) + (size_t)md[1] * ((size_t)q[2] << sh))];
-            if (j >= 0 && b->meta_h[j].level == L) {
+            int j = leaf(o);
+            if (j >= 0) {
               row[s] = b->meta_h[j].base;
-            } else {
-              // computed here: the entry cell_at() shifts back into this block
-              row[s] = mi.base + (int64_t)ox * mi.nx + (int64_t)mi.PX * ((int64_t)oy * mi.ny + (int64_t)mi.NY * oz * mi.nz);
-              local |= 1u << s;
+              any = true;
+              continue;
             }
+            // An edge or corner sector with a leaf of this level beside it
+            // (at o without the component d) is that leaf's face sector along
+            // d, which that leaf computes: read from its guard cells.  Where
+            // a layer of leaves meets coarser ones, every leaf computed its
+            // face sector and the 8 around it, 28 x 28 x 6 cells of 16^3
+            // blocks in the first stage instead of 16 x 16 x 6.
+            for (int d = 0; d < 3 && j < 0; d++) {
+              if (o[d] == 0 || (ox != 0) + (oy != 0) + (oz != 0) < 2) continue;
+              int t[3] = {ox, oy, oz}, f[3] = {0, 0, 0};
+              t[d] = 0;
+              f[d] = o[d];
+              j = leaf(t);
+              if (j >= 0) row[s] = b->meta_h[j].base + shift(f);
+            }
+            if (j >= 0) continue;
+            // computed here: the entry cell_at() shifts back into this block
+            row[s] = mi.base + shift(o);
+            local |= 1u << s;
           }
-      if (local == all_sectors) continue;  // telescopes over its own guard cells
+      if (!any) continue;  // telescopes over its own guard cells
       std::copy(row, row + 27, nb.begin() + (size_t)i * 27);
       b->amr_local[i] = local;
       b->amr_remap_blk[i] = local ? 2 : 1;
