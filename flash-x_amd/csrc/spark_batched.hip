@@ -1,14 +1,12 @@
 // spark_batched.hip -- the batched form of the Spark RK stage: one fused,
 // persistent launch per RK stage over every block of the batch.
 //
-// This file is compiled twice:
-//   SPARK_FUSED_REAL=float   FP32 reconstruction / Riemann arithmetic
-//                            (the FP32-flux form, -ffp-contract=fast)
-//   SPARK_FUSED_REAL=double  FP64 throughout, every expression in the
-//                            reference's order (-ffp-contract=off), so it
-//                            reproduces the plain FP64 form bit for bit
-// Conserved-variable accumulation, floors, EOS and flux-register sums are
-// FP64 in both.
+// This is the FP32-flux form: FP32 reconstruction and Riemann arithmetic
+// (built with -ffp-contract=fast); conserved-variable accumulation, floors,
+// EOS and flux-register sums are FP64.  (The same kernel in FP64 needed ~330
+// registers, one wave per SIMD: 8 steps of 360 leaves of 16^3 with 8 scalars on
+// three levels took 65 ms against 33 ms in the directional sweeps of
+// spark_plain.hip, which run the batched FP64 form instead.)
 //
 // Work items are (block, x-y tile); a workgroup takes items from per-XCD
 // queues (an XCD's queue holds whole blocks, so the halos that tiles of one
@@ -33,33 +31,21 @@
 // reference order (x, y, z, source; hy_rk_updateSoln.F90-mc:257-265).
 // Stage input and output states are distinct buffers, so no tile reads a
 // cell another tile writes.
-#include <type_traits>
-
 #include "spark_physics.hpp"
 #include "spark_batched.hpp"
-
-#ifndef SPARK_FUSED_REAL
-#define SPARK_FUSED_REAL float
-#endif
-
-#define FUSED_NAME2(a, b) a##b
-#define FUSED_NAME(a, b) FUSED_NAME2(a, b)
-#define FUSED_SFX SPARK_FUSED_SUFFIX
 
 namespace spark {
 namespace {
 
-using Real = SPARK_FUSED_REAL;
-constexpr bool kF64 = std::is_same<Real, double>::value;
+using Real = float;
 constexpr int NT = FUSED_THREADS;
-// hydro slots staged per cell: dens velx vely velz pres [gamc] rhoe.  The
-// FP32 form takes gamc = gamma (the Gamma EOS sets every cell's gamc to
+// hydro slots staged per cell: dens velx vely velz pres rhoe.  The form takes gamc = gamma (the Gamma EOS sets every cell's gamc to
 // gamma), so it neither stages nor reconstructs it.
-constexpr int NH = kF64 ? 7 : 6;
+constexpr int NH = 6;
 constexpr int CH = FUSED_SCALAR_CHUNK;  // mass scalars per chunk (the species all in the first)
 constexpr int SL_RHOE = NH - 1;
 
-__host__ __device__ __forceinline__ constexpr int hslot(int s) { return (!kF64 && s >= R_GAMC) ? s + 1 : s; }
+__host__ __device__ __forceinline__ constexpr int hslot(int s) { return s >= R_GAMC ? s + 1 : s; }
 __host__ __device__ __forceinline__ constexpr int rup64(int n) { return (n + 63) & ~63; }
 
 // LDS carve-up of one work item, in Reals
@@ -101,7 +87,7 @@ __device__ __forceinline__ int fquot(int w, const FDiv& f, int& r) {
 }
 
 // staged slot v of cell c: hydro slots in the pencil order, then scalars
-__device__ __forceinline__ Real load_slot(const double* __restrict__ s, int64_t cs, int64_t c, int v, double gamma) {
+__device__ __forceinline__ Real load_slot(const double* __restrict__ s, int64_t cs, int64_t c, int v) {
   if (v >= NH) return (Real)s[(V_NPROP + v - NH) * cs + c];
   switch (hslot(v)) {
     case R_DENS: return (Real)s[V_DENS * cs + c];
@@ -109,7 +95,6 @@ __device__ __forceinline__ Real load_slot(const double* __restrict__ s, int64_t 
     case R_VELY: return (Real)s[V_VELY * cs + c];
     case R_VELZ: return (Real)s[V_VELZ * cs + c];
     case R_PRES: return (Real)s[V_PRES * cs + c];
-    case R_GAMC: return kF64 ? (Real)s[V_GAMC * cs + c] : (Real)gamma;
     default: return (Real)(s[V_DENS * cs + c] * s[V_EINT * cs + c]);
   }
 }
@@ -154,7 +139,8 @@ __device__ __forceinline__ void hydro_face(const RParams& rp, Real* L, Real* R, 
   L[R_PRES] = fmax2(rp.smallp, L[R_PRES]);
   R[R_DENS] = fmax2(rp.smlrho, R[R_DENS]);
   R[R_PRES] = fmax2(rp.smallp, R[R_PRES]);
-  if (!kF64) { L[R_GAMC] = rp.gamma; R[R_GAMC] = rp.gamma; }
+  L[R_GAMC] = rp.gamma;
+  R[R_GAMC] = rp.gamma;
   int ierr;
   if (RIEMANN == RIEMANN_HLL) ierr = hll<DIR, Real>(L, R, F);
   else ierr = hllc<DIR, Real>(L, R, RIEMANN == RIEMANN_HLLC_HYBRID, inShock, rp.tiny, F);
@@ -182,7 +168,8 @@ __device__ __forceinline__ void face_states(const Real* __restrict__ bp, const R
     L[hslot(s)] = bp[s * nr + il];
     R[hslot(s)] = bm[s * nr + ir];
   }
-  if (!kF64) { L[R_GAMC] = Real(0.); R[R_GAMC] = Real(0.); }
+  L[R_GAMC] = Real(0.);
+  R[R_GAMC] = Real(0.);
 }
 
 // species face states: clamp to [smallx, 1] and renormalise, left and right
@@ -282,24 +269,9 @@ __device__ __forceinline__ void xy_face(const FusedArgs& A, const BlockMeta& m, 
   }
 }
 
+// two waves per SIMD: <= 256 VGPRs, no spills, with or without scalars
 template <int NSM, int RECON, int RIEMANN>
-// waves per SIMD the register allocation targets: the FP32 form fits 2
-// (<= 256 VGPRs, no spills, with or without scalars); the FP64 form keeps
-// all its registers (accumulation registers included) at 1 rather than
-// spilling
-#ifndef FUSED_WAVES_OF
-#define FUSED_WAVES_OF(nsm) (kF64 ? 1 : 2)
-#endif
-#ifndef FUSED_XY_UNROLL
-#define FUSED_XY_UNROLL 6
-#endif
-#ifndef FUSED_EARLY_Z
-#define FUSED_EARLY_Z kF64
-#endif
-#ifndef EARLY_Z_BARRIER
-#define EARLY_Z_BARRIER
-#endif
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_WAVES_OF(NSM)))) FUSED_NAME(k_fused, FUSED_SFX)(FusedArgs A) {
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) k_fused_f32(FusedArgs A) {
   constexpr int NFM = F_NUM + NSM;
   constexpr int NSA = NSM > 0 ? NSM : 1;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -393,7 +365,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
       for (int w = 1; w < 5; w++) {
         const int64_t c = cell_at(m, nbt, g, ci, cj, I.z0 - 4 + w);
 #pragma unroll
-        for (int v = 0; v < NH; v++) win[v][w] = load_slot(S, cs, c, v, P.gamma);
+        for (int v = 0; v < NH; v++) win[v][w] = load_slot(S, cs, c, v);
       }
     }
 
@@ -406,7 +378,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
         for (int v = 0; v < NH; v++) {
 #pragma unroll
           for (int w = 0; w < 4; w++) win[v][w] = win[v][w + 1];
-          win[v][4] = load_slot(S, cs, c, v, P.gamma);
+          win[v][4] = load_slot(S, cs, c, v);
           plane[v * psz + pcc] = win[v][2];
         }
         // scalars: the plane only (their z stencils are read again when the
@@ -443,7 +415,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
           // the first of its stores waits
           Real hv[NH > NSA ? NH : NSA];
 #pragma unroll
-          for (int v = 0; v < NH; v++) hv[v] = load_slot(S, cs, c, v, P.gamma);
+          for (int v = 0; v < NH; v++) hv[v] = load_slot(S, cs, c, v);
 #pragma unroll
           for (int v = 0; v < NH; v++) plane[v * psz + pc] = hv[v];
           // (slots past ns load scalar ns-1 again, so no load is conditional)
@@ -474,7 +446,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
             else { const int r = h - 2 * (tx + 2); py = 1 + r / 2; px = (r & 1) ? tx + 1 : 0; }
           }
           const int pc = (py + 2) * PW + (px + 2);
-          const Real g0 = kF64 ? plane[R_GAMC * psz + pc] : rp.gamma;
+          const Real g0 = rp.gamma;
           const Real fx = flat_dir(pp[pc - 2], pp[pc - 1], pp[pc], pp[pc + 1], pp[pc + 2], g0, plane[1 * psz + pc],
                                    plane[1 * psz + pc + 1]);
           const Real fy = flat_dir(pp[pc - 2 * PW], pp[pc - PW], pp[pc], pp[pc + PW], pp[pc + 2 * PW], g0,
@@ -522,7 +494,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
           else { ry = fquot(w, d_tx, rx) - 1; st = PW; nr = nry; om = ym; op = yp; }
           const int pc = (ry + 3) * PW + (rx + 3);
           const Real fl = use_flat ? flatb[(ry + 1) * (tx + 2) + (rx + 1)] : Real(1.);
-#pragma unroll FUSED_XY_UNROLL
+#pragma unroll
           for (int v = 0; v < NH; v++) {
             const Real* r = plane + v * psz + pc;
             const Real u5[5] = {r[-2 * st], r[-st], r[0], r[st], r[2 * st]};
@@ -551,7 +523,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
                 Ls[hslot(s)] = upz[s];
                 Rs[hslot(s)] = umz[s];
               }
-              if (!kF64) { Ls[R_GAMC] = Real(0.); Rs[R_GAMC] = Real(0.); }
+              Ls[R_GAMC] = Real(0.);
+              Rs[R_GAMC] = Real(0.);
               cl[0] = win[0][1]; cl[1] = win[1][1]; cl[2] = win[2][1]; cl[3] = win[3][1]; cl[4] = win[SL_RHOE][1];
               cr[0] = win[0][2]; cr[1] = win[1][2]; cr[2] = win[2][2]; cr[3] = win[3][2]; cr[4] = win[SL_RHOE][2];
               bool shk = false;
@@ -583,10 +556,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
       // ---- P5: update of level k-1 (hydro part), x/y differences of level k
       const bool upd = col && k - 1 >= I.z0 && k - 1 <= I.z1;
       double d0 = 0., ds = 0., dens1 = 1.;
-      // Multigamma (FP64 form): the EOS of level k-1 waits for its updated
-      // species (first scalar chunk); dens vx vy vz ener eint meanwhile
-      const bool defer_eos = kF64 && P.eos == 1;
-      double mg[6] = {0., 0., 0., 0., 0., 0.};
       if (upd) {
         // FP64 (hy_rk_updateSoln.F90-mc:227-287)
         const int64_t c = colc + (int64_t)(k - 1) * sz;
@@ -627,18 +596,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
         sout[V_VELX * cs + c] = vx;
         sout[V_VELY * cs + c] = vy;
         sout[V_VELZ * cs + c] = vz;
-        if (defer_eos) {
-          mg[0] = dens; mg[1] = vx; mg[2] = vy; mg[3] = vz; mg[4] = ener; mg[5] = eint;
-        } else {
-          EosOut e = eos_dens_ei(P, dens, vx, vy, vz, ener, eint);
-          sout[V_PRES * cs + c] = e.pres;
-          sout[V_GAMC * cs + c] = P.gamma;
-          sout[V_EINT * cs + c] = e.eint;
-          sout[V_ENER * cs + c] = e.ener;
-          if (A.final_stage) {
-            sout[V_TEMP * cs + c] = e.temp;
-            sout[V_GAME * cs + c] = e.game;
-          }
+        EosOut e = eos_dens_ei(P, dens, vx, vy, vz, ener, eint);
+        sout[V_PRES * cs + c] = e.pres;
+        sout[V_GAMC * cs + c] = P.gamma;
+        sout[V_EINT * cs + c] = e.eint;
+        sout[V_ENER * cs + c] = e.ener;
+        if (A.final_stage) {
+          sout[V_TEMP * cs + c] = e.temp;
+          sout[V_GAME * cs + c] = e.game;
         }
         dens1 = dens;
       }
@@ -672,37 +637,24 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
             const int nrxp = rup64(nrx);
             const int utot = Cp + (xyk ? nrxp + nry : 0);
             // the column's z stencils (task u = tid < C); a slot past nc
-            // loads scalar nc-1 again.  The FP64 form loads them first and
-            // runs the thread's x/y tasks (u >= Cp, stencils in LDS) while
-            // they are in flight; the FP32 form (two waves per SIMD, no
-            // registers to spare) loads and reconstructs them in its column
-            // task
+            // loads scalar nc-1 again
             Real u5s[CH][5];
-            auto load_z = [&]() {
-              int64_t zc[5];
-#pragma unroll
-              for (int w = 0; w < 5; w++) zc[w] = cell_at(m, nbt, g, ci, cj, k - 2 + w);
-#pragma unroll
-              for (int j = 0; j < CH; j++) {
-                const double* sp = S + (int64_t)(V_NPROP + c0 + (j < nc ? j : nc - 1)) * cs;
-#pragma unroll
-                for (int w = 0; w < 5; w++) u5s[j][w] = (Real)sp[zc[w]];
-              }
-              EARLY_Z_BARRIER;
-            };
-            auto recon_z = [&]() {
-              const Real fl = use_flat ? flatb[fcc] : Real(1.);
-#pragma unroll
-              for (int j = 0; j < CH; j++)
-                if (j < nc) recon1<RECON, Real>(u5s[j], fl, upsk[j], ums[j]);
-            };
-            constexpr bool early = FUSED_EARLY_Z;
-            if (early && col) load_z();
-            for (int u = early && tid < Cp ? tid + NT : tid; u < utot; u += NT) {
+            for (int u = tid; u < utot; u += NT) {
               if (u < Cp) {
                 if (u < C) {
-                  load_z();
-                  recon_z();
+                  int64_t zc[5];
+#pragma unroll
+                  for (int w = 0; w < 5; w++) zc[w] = cell_at(m, nbt, g, ci, cj, k - 2 + w);
+#pragma unroll
+                  for (int j = 0; j < CH; j++) {
+                    const double* sp = S + (int64_t)(V_NPROP + c0 + (j < nc ? j : nc - 1)) * cs;
+#pragma unroll
+                    for (int w = 0; w < 5; w++) u5s[j][w] = (Real)sp[zc[w]];
+                  }
+                  const Real fl = use_flat ? flatb[fcc] : Real(1.);
+#pragma unroll
+                  for (int j = 0; j < CH; j++)
+                    if (j < nc) recon1<RECON, Real>(u5s[j], fl, upsk[j], ums[j]);
                 }
                 continue;
               }
@@ -725,7 +677,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
                 op[j * nr + w] = up;
               }
             }
-            if (early && col) recon_z();
           }
           __syncthreads();
           // S2: upwinded scalar fluxes
@@ -811,7 +762,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
           // S3: scalar update of level k-1, x/y differences of level k
           if (upd) {
             const int64_t c = colc + (int64_t)(k - 1) * sz;
-            double Xn[8] = {0., 0., 0., 0., 0., 0., 0., 0.};  // updated species of the first chunk
             // the chunk's U0 and stage-input loads issue before the first
             // store (which the compiler cannot tell apart from them); a slot
             // past nc re-reads scalar nc-1
@@ -833,20 +783,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FUSED_W
                 Bu = A.c1 * Au + A.c2 * Bu + A.c3 * inner_n;
                 const double x = Bu / dens1;
                 sout[(V_NPROP + c0 + j) * cs + c] = x;
-                if (c0 == 0) Xn[j] = x;
-              }
-            }
-            if (defer_eos && c0 == 0) {
-              // the EOS of level k-1 with its updated species (Eos_wrapped
-              // after updateSoln)
-              const EosOut e = eos_dens_ei(P, mg[0], mg[1], mg[2], mg[3], mg[4], mg[5], Xn);
-              sout[V_PRES * cs + c] = e.pres;
-              sout[V_GAMC * cs + c] = e.gamc;
-              sout[V_EINT * cs + c] = e.eint;
-              sout[V_ENER * cs + c] = e.ener;
-              if (A.final_stage) {
-                sout[V_TEMP * cs + c] = e.temp;
-                sout[V_GAME * cs + c] = e.game;
               }
             }
           }
@@ -878,7 +814,7 @@ __global__ void k_reset_counters(int* c, int n) {
 
 template <int NSM, int RECON, int RIEMANN>
 hipError_t launch_t(const FusedArgs& A, int grid, size_t lds, hipStream_t st) {
-  hipLaunchKernelGGL((FUSED_NAME(k_fused, FUSED_SFX)<NSM, RECON, RIEMANN>), dim3(grid), dim3(FUSED_THREADS), lds, st,
+  hipLaunchKernelGGL((k_fused_f32<NSM, RECON, RIEMANN>), dim3(grid), dim3(FUSED_THREADS), lds, st,
                      A);
   return hipGetLastError();
 }
@@ -902,36 +838,36 @@ hipError_t launch_r(const FusedArgs& A, int grid, size_t lds, hipStream_t st) {
 
 }  // namespace
 
-size_t FUSED_NAME(fused_lds_bytes, FUSED_SFX)(int ns, int tx, int ty) {
+size_t fused_lds_bytes(int ns, int tx, int ty) {
   return sizeof(Real) * (size_t)lds_layout(tx, ty, NH + ns).total;
 }
 
-hipError_t FUSED_NAME(fused_reset, FUSED_SFX)(hipStream_t st, int* counters) {
+hipError_t fused_reset(hipStream_t st, int* counters) {
   hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, counters, FUSED_XCDS);
   return hipGetLastError();
 }
 
-hipError_t FUSED_NAME(fused_stage, FUSED_SFX)(const FusedArgs& A, int grid, size_t lds, hipStream_t st) {
+hipError_t fused_stage(const FusedArgs& A, int grid, size_t lds, hipStream_t st) {
   return (A.P.ns == 0) ? launch_r<0>(A, grid, lds, st) : launch_r<8>(A, grid, lds, st);
 }
 
-hipError_t FUSED_NAME(fused_occupancy, FUSED_SFX)(int ns, size_t lds, int* blocks_per_cu) {
+hipError_t fused_occupancy(int ns, size_t lds, int* blocks_per_cu) {
   if (ns == 0)
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        blocks_per_cu, FUSED_NAME(k_fused, FUSED_SFX)<0, RECON_WENO5, RIEMANN_HLLC>, FUSED_THREADS, lds);
+        blocks_per_cu, k_fused_f32<0, RECON_WENO5, RIEMANN_HLLC>, FUSED_THREADS, lds);
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      blocks_per_cu, FUSED_NAME(k_fused, FUSED_SFX)<8, RECON_WENO5, RIEMANN_HLLC>, FUSED_THREADS, lds);
+      blocks_per_cu, k_fused_f32<8, RECON_WENO5, RIEMANN_HLLC>, FUSED_THREADS, lds);
 }
 
 // static LDS of the kernel (work-item index, neighbour table): a launch's
 // dynamic LDS must leave room for it under the per-workgroup limit
-size_t FUSED_NAME(fused_static_lds, FUSED_SFX)(int ns) {
+size_t fused_static_lds(int ns) {
   hipFuncAttributes fa;
   hipError_t e = ns == 0
                      ? hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(
-                                                     FUSED_NAME(k_fused, FUSED_SFX)<0, RECON_WENO5, RIEMANN_HLLC>))
+                                                     k_fused_f32<0, RECON_WENO5, RIEMANN_HLLC>))
                      : hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(
-                                                     FUSED_NAME(k_fused, FUSED_SFX)<8, RECON_WENO5, RIEMANN_HLLC>));
+                                                     k_fused_f32<8, RECON_WENO5, RIEMANN_HLLC>));
   const size_t own = sizeof(int) + 27 * sizeof(int64_t);
   if (e != hipSuccess) return 1024;  // a safe upper bound of the kernel's own variables
   return fa.sharedSizeBytes > own ? fa.sharedSizeBytes : own;

@@ -87,17 +87,12 @@ struct FusedArgs {
   int* err;
 };
 
-// the fused stage kernel in FP32 (_f32) and FP64 (_f64) arithmetic; the LDS
+// the fused stage kernel (FP32 flux arithmetic); the LDS
 // of a work item depends on its tile (tx x ty, tx * ty <= FUSED_THREADS)
-size_t fused_lds_bytes_f32(int ns, int tx, int ty);
-hipError_t fused_reset_f32(hipStream_t st, int* counters);
-hipError_t fused_stage_f32(const FusedArgs& A, int grid, size_t lds, hipStream_t st);
-hipError_t fused_occupancy_f32(int ns, size_t lds, int* blocks_per_cu);
-size_t fused_static_lds_f32(int ns);  // the kernel's own __shared__ bytes beside the dynamic LDS
-size_t fused_lds_bytes_f64(int ns, int tx, int ty);
-hipError_t fused_reset_f64(hipStream_t st, int* counters);
-hipError_t fused_stage_f64(const FusedArgs& A, int grid, size_t lds, hipStream_t st);
-hipError_t fused_occupancy_f64(int ns, size_t lds, int* blocks_per_cu);
-size_t fused_static_lds_f64(int ns);
+size_t fused_lds_bytes(int ns, int tx, int ty);
+hipError_t fused_reset(hipStream_t st, int* counters);
+hipError_t fused_stage(const FusedArgs& A, int grid, size_t lds, hipStream_t st);
+hipError_t fused_occupancy(int ns, size_t lds, int* blocks_per_cu);
+size_t fused_static_lds(int ns);  // the kernel's own __shared__ bytes beside the dynamic LDS
 
 }  // namespace spark

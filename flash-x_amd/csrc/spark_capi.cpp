@@ -20,6 +20,7 @@
 #include <cstring>
 #include <exception>
 #include <map>
+#include <set>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -102,8 +103,9 @@ struct spark_batch {
   // of the last stage run before the final one (spark_unpack which = 1)
   double* S2 = nullptr;
   double* star = nullptr;
-  bool fused = false;
-  bool fused64 = false;  // batched form in FP64 arithmetic
+  bool fused = false;     // FP32-flux form: the persistent stage kernel
+  // a batched form: its stages read same-level halos wherever they run from
+  bool batched = false;
   int cus = 0;            // compute units of the device
   size_t lds_limit = 0;   // LDS bytes a workgroup may allocate
   int64_t* nbr_d = nullptr;  // uniform grid: 27 neighbour pool offsets per block
@@ -331,7 +333,7 @@ int run_exchange(spark_batch* b) {
 int run_amr_correct(spark_batch* b) {
   int rc;
   if ((rc = run_exchange(b))) return rc;
-  if (b->fused && !b->fused64) {
+  if (b->fused) {
     // FP32-flux form: only the cells on a face toward a finer leaf (their
     // whole x, y, z sequence).  Everywhere else the correction is zero and
     // the reference's pass is the identity up to one FP64 rounding of the
@@ -372,7 +374,7 @@ int run_step_begin(spark_batch* b, bool same_level = false) {
   // own in the stages) get it one layer out.
   const bool hyb = b->p.use_hybrid_riemann != 0;
   const int band = !hyb ? 0 : (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + 1;
-  if (amr_remap_on(b) && (b->fused || same_level)) {
+  if (amr_remap_on(b) && (b->batched || same_level)) {
     // a hierarchy has one block shape
     PlainLaunch L = make_launch(b, b->classes[0]);
     if (b->n_tele > 0) {
@@ -427,24 +429,22 @@ int fused_plan(spark_batch* b);
 int fused_tune(spark_batch* b);
 
 size_t fused_lds(const spark_batch* b, int tx, int ty) {
-  return b->fused64 ? spark::fused_lds_bytes_f64(b->p.nscalars, tx, ty)
-                    : spark::fused_lds_bytes_f32(b->p.nscalars, tx, ty);
+  return spark::fused_lds_bytes(b->p.nscalars, tx, ty);
 }
 
 // persistent grid for a given LDS size: resident workgroups of the whole
 // device, a multiple of the XCD count
 int fused_grid_for(const spark_batch* b, size_t lds) {
   int occ = 0;
-  hipError_t e = b->fused64 ? spark::fused_occupancy_f64(b->p.nscalars, lds, &occ)
-                            : spark::fused_occupancy_f32(b->p.nscalars, lds, &occ);
+  hipError_t e = spark::fused_occupancy(b->p.nscalars, lds, &occ);
   if (e != hipSuccess || occ < 1) occ = 1;
   return std::max(spark::FUSED_XCDS, (b->cus * occ) / spark::FUSED_XCDS * spark::FUSED_XCDS);
 }
 
 hipError_t fused_launch(const spark_batch* b, const spark::FusedArgs& A, int grid, size_t lds) {
-  hipError_t e = b->fused64 ? spark::fused_reset_f64(g_stream, A.counters) : spark::fused_reset_f32(g_stream, A.counters);
+  hipError_t e = spark::fused_reset(g_stream, A.counters);
   if (e != hipSuccess) return e;
-  return b->fused64 ? spark::fused_stage_f64(A, grid, lds, g_stream) : spark::fused_stage_f32(A, grid, lds, g_stream);
+  return spark::fused_stage(A, grid, lds, g_stream);
 }
 
 // 3D blocks of a uniform grid in refill mode read halo cells from the
@@ -481,15 +481,42 @@ spark::FusedArgs fused_args(spark_batch* b, int stage) {
   return A;
 }
 
+// one stage of the sweeps on a hierarchy over the boxes of its groups
+int run_stage_groups(spark_batch* b, int stage) {
+  const double* co = b->coeff[stage - 1];
+  double* out = stage_out(b, stage);
+  if (stage != b->last_stage) b->star = out;
+  PlainLaunch L = make_launch(b, b->classes[0]);
+  L.weight = b->weights[stage - 1];
+  L.add_flux = stage > 1;
+  L.Sin = stage_in(b, stage);
+  L.Sout = out;
+  for (const auto& g : b->groups[stage - 1]) {
+    PlainLaunch G = L;
+    G.blist = g.ids_d;
+    G.blo = g.lo_d;
+    G.nbr = b->nbr_d;
+    G.nblk = g.n;
+    for (int d = 0; d < 3; d++) {
+      G.ext[d] = g.ext[d];
+      if (!g.interior) G.fb[d] = nullptr;
+    }
+    HIPCHK(spark::plain_stage(G, 0, co[0], co[1], co[2], stage == b->last_stage));
+  }
+  return SPARK_OK;
+}
+
 // saveState's copy is folded away: stage 1 reads the solution U directly
 // (hy_starState == Uin at stage 1) and the last stage writes U directly
 // (updateState copies exactly the last stage's region, the interior).
 int run_stage(spark_batch* b, int stage, int ngoff, bool same_level = false) {
+  if (b->batched && ngoff != stage_ngoff(b, stage))
+    return fail(SPARK_ERR_ARG, "batched form: stage %d runs with ngoff %d", stage, stage_ngoff(b, stage));
+  same_level = same_level || b->batched;
+  if (!b->fused && same_level && amr_remap_on(b)) return run_stage_groups(b, stage);
   const double* co = b->coeff[stage - 1];
   if (stage != b->last_stage) b->star = stage_out(b, stage);
   if (b->fused) {
-    if (ngoff != stage_ngoff(b, stage))
-      return fail(SPARK_ERR_ARG, "batched form: stage %d runs with ngoff %d", stage, stage_ngoff(b, stage));
     int rc;
     if (!b->planned && (rc = fused_plan(b))) return rc;
     spark::FusedArgs A = fused_args(b, stage);
@@ -516,31 +543,6 @@ int run_stage(spark_batch* b, int stage, int ngoff, bool same_level = false) {
   return SPARK_OK;
 }
 
-// one stage of the plain form on a hierarchy over the boxes of its groups
-int run_stage_groups(spark_batch* b, int stage) {
-  const double* co = b->coeff[stage - 1];
-  double* out = stage_out(b, stage);
-  if (stage != b->last_stage) b->star = out;
-  PlainLaunch L = make_launch(b, b->classes[0]);
-  L.weight = b->weights[stage - 1];
-  L.add_flux = stage > 1;
-  L.Sin = stage_in(b, stage);
-  L.Sout = out;
-  for (const auto& g : b->groups[stage - 1]) {
-    PlainLaunch G = L;
-    G.blist = g.ids_d;
-    G.blo = g.lo_d;
-    G.nbr = b->nbr_d;
-    G.nblk = g.n;
-    for (int d = 0; d < 3; d++) {
-      G.ext[d] = g.ext[d];
-      if (!g.interior) G.fb[d] = nullptr;
-    }
-    HIPCHK(spark::plain_stage(G, 0, co[0], co[1], co[2], stage == b->last_stage));
-  }
-  return SPARK_OK;
-}
-
 int run_step_end(spark_batch* b) {
   b->step_open = false;
   return SPARK_OK;
@@ -549,11 +551,6 @@ int run_step_end(spark_batch* b) {
 int run_full_step(spark_batch* b) {
   int rc;
   if ((rc = run_step_begin(b, true))) return rc;
-  if (!b->fused && amr_remap_on(b)) {
-    for (int s = 1; s <= b->last_stage; s++)
-      if ((rc = run_stage_groups(b, s))) return rc;
-    return run_step_end(b);
-  }
   const bool refill = b->p.guard_mode == SPARK_GUARD_REFILL;
   for (int s = 1; s <= b->last_stage; s++) {
     if ((rc = run_stage(b, s, refill ? 0 : b->limits_array[s - 1], true))) return rc;
@@ -975,7 +972,8 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   if (p->form == SPARK_FORM_FP32_FLUX || p->form == SPARK_FORM_BATCHED_FP64) {
     if (p->ndim != 3) return fail(SPARK_ERR_ARG, "the batched form is 3D only (ndim = %d)", p->ndim);
     // species are clamped and renormalised together, within the first
-    // chunk of scalars the fused kernel stages
+    // chunk of scalars the fused kernel stages (both batched forms take the
+    // same number)
     if (p->nspecies > spark::FUSED_SCALAR_CHUNK)
       return fail(SPARK_ERR_ARG, "the batched forms take at most %d species (nspecies = %d)",
                   spark::FUSED_SCALAR_CHUNK, p->nspecies);
@@ -1090,10 +1088,9 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   ALLOC(b->S, sizeof(double) * b->pool);
   ALLOC(b->flat, sizeof(double) * b->opool);
   ALLOC(b->S2, sizeof(double) * b->pool);
-  // the plain form's divergence terms (the sweeps before the last write
+  // the divergence terms of the sweeps (the sweeps before the last write
   // them; 1D has no earlier sweep)
-  const bool plain_form = p->form != SPARK_FORM_FP32_FLUX && p->form != SPARK_FORM_BATCHED_FP64;
-  if (plain_form && p->ndim > 1) ALLOC(b->div, sizeof(double) * b->dpool);
+  if (p->form != SPARK_FORM_FP32_FLUX && p->ndim > 1) ALLOC(b->div, sizeof(double) * b->dpool);
   if (p->flux_correct) {
     for (int q = 0; q < 3; q++) ALLOC(b->fb[q], sizeof(double) * b->bpool);
     for (int q = 0; q < 3; q++) ALLOC(b->fc[q], sizeof(double) * b->bpool);
@@ -1116,9 +1113,9 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   ALLOC(b->dtparts, spark::plain_dt_part_size() * (size_t)nblocks * b->dtchunks);
   ALLOC(b->err, sizeof(int));
   ALLOC(b->hist_slot, sizeof(int));
-  if (p->form == SPARK_FORM_FP32_FLUX || p->form == SPARK_FORM_BATCHED_FP64) {
+  b->batched = p->form == SPARK_FORM_FP32_FLUX || p->form == SPARK_FORM_BATCHED_FP64;
+  if (p->form == SPARK_FORM_FP32_FLUX) {
     b->fused = true;
-    b->fused64 = p->form == SPARK_FORM_BATCHED_FP64;
     ALLOC(b->counters, sizeof(int) * 3 * spark::FUSED_XCDS);
     ALLOC(b->tune_err, sizeof(int));
     ALLOC(b->tune_dt, sizeof(double));
@@ -1144,7 +1141,7 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
     HIPCHK(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, g_device));
     HIPCHK(hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, g_device));
     // the dynamic LDS of a launch plus the kernel's own __shared__ variables
-    const size_t own = b->fused64 ? spark::fused_static_lds_f64(b->p.nscalars) : spark::fused_static_lds_f32(b->p.nscalars);
+    const size_t own = spark::fused_static_lds(b->p.nscalars);
     b->lds_limit = (size_t)lim > own + 16 ? (size_t)lim - own - 16 : 0;
     if (fused_lds(b, 4, 4) > b->lds_limit) {
       const size_t need = fused_lds(b, 4, 4), have = b->lds_limit;
@@ -1262,7 +1259,7 @@ int spark_set_uniform_grid(spark_batch* b, int nbx, int nby, int nbz) {
   if (b->amr) return fail(SPARK_ERR_STATE, "spark_set_uniform_grid: the batch has a block hierarchy");
   if ((b->p.ndim < 2 && nby != 1) || (b->p.ndim < 3 && nbz != 1))
     return fail(SPARK_ERR_ARG, "uniform grid extent in an unused dimension");
-  if (b->fused && b->p.guard_mode == SPARK_GUARD_REFILL) {
+  if (b->batched && b->p.guard_mode == SPARK_GUARD_REFILL) {
     const BlockMeta& m0 = b->meta_h[0];
     if (m0.nx < 3 || m0.ny < 3 || m0.nz < 3)
       return fail(SPARK_ERR_ARG, "batched form on a uniform grid needs blocks of >= 3 cells per side");
@@ -1420,7 +1417,7 @@ int spark_set_geometry(spark_batch* b, int geometry, const double* const* r_cent
   }
   if (geometry != SPARK_GEOM_CYLINDRICAL && geometry != SPARK_GEOM_SPHERICAL)
     return fail(SPARK_ERR_ARG, "spark_set_geometry: geometry %d", geometry);
-  if (b->fused) return fail(SPARK_ERR_ARG, "spark_set_geometry: the batched forms are Cartesian only");
+  if (b->batched) return fail(SPARK_ERR_ARG, "spark_set_geometry: the batched forms are Cartesian only");
   // the hierarchy's prolongation and flux restriction are the Cartesian ones
   if (b->amr) return fail(SPARK_ERR_STATE, "spark_set_geometry: the block hierarchy is Cartesian only");
   // the Grid's cell volumes exist for cylindrical geometry in 2D and
@@ -1506,7 +1503,25 @@ int spark_set_option(spark_batch* b, int option, int value) {
 
 int spark_batched_tiles(spark_batch* b, int* out, int max_rows, int* nrows) {
   if (!b || !out || !nrows) return fail(SPARK_ERR_ARG, "spark_batched_tiles: bad argument");
-  if (!b->fused) return fail(SPARK_ERR_STATE, "spark_batched_tiles: not a batched FP32-flux batch");
+  if (!b->batched) return fail(SPARK_ERR_STATE, "spark_batched_tiles: not a batched FP32-flux batch");
+  if (!b->fused) {
+    // the sweeps cover whole regions: their cross-sections, per shape and depth
+    std::set<std::tuple<int, int, int, int>> rows;
+    for (const auto& c : b->classes)
+      for (int s = 1; s <= b->last_stage; s++) rows.insert(std::make_tuple(c.nx, c.ny, c.nz, stage_ngoff(b, s)));
+    int n = 0;
+    for (const auto& t : rows) {
+      if (n < max_rows) {
+        int* r = out + 6 * n;
+        std::tie(r[0], r[1], r[2], r[3]) = t;
+        r[4] = r[0] + 2 * r[3];
+        r[5] = r[1] + 2 * r[3];
+      }
+      n++;
+    }
+    *nrows = n;
+    return SPARK_OK;
+  }
   int rc;
   if (!b->planned && (rc = fused_plan(b))) return rc;
   int n = 0;
