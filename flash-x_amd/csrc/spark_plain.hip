@@ -419,7 +419,9 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
       else if (v <= R_VELZ) sm[(R_NUM + v) * NT + tid] = cur[2];
       else if (v == R_RHOE) sm[(R_NUM + 4) * NT + tid] = cur[2];
     }
-    sm[(R_NUM + 5) * NT + tid] = Ushok[m.base + V_SHOK * cs + c];
+    // only the hybrid solver reads SHOK (one of the 16 fields a sweep would
+    // otherwise fetch)
+    if (P.hybrid) sm[(R_NUM + 5) * NT + tid] = Ushok[m.base + V_SHOK * cs + c];
   }
   __syncthreads();
   const bool face = valid && s >= 1;
@@ -436,7 +438,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
     left[R_PRES] = fmax2(P.smallp, left[R_PRES]);
     right[R_DENS] = fmax2(P.smlrho, right[R_DENS]);
     right[R_PRES] = fmax2(P.smallp, right[R_PRES]);
-    const bool inShock = (sm[(R_NUM + 5) * NT + tn] != 0.0) || (sm[(R_NUM + 5) * NT + tid] != 0.0);
+    const bool inShock = P.hybrid && (sm[(R_NUM + 5) * NT + tn] != 0.0 || sm[(R_NUM + 5) * NT + tid] != 0.0);
     int ierr;
     if (RIEMANN == RIEMANN_HLL) ierr = hll<DIR, double>(left, right, F);
     else ierr = hllc<DIR, double>(left, right, P.hybrid != 0, inShock, P.tiny, F);
@@ -1212,6 +1214,11 @@ static hipError_t launch_sweeps(const PlainLaunch& L, int ngoff, const UpdArgs& 
   return launch_flux_r<2, NSM, 3, NB>(L, ngoff, UA);
 }
 
+template <int NSM>
+static hipError_t launch_sweeps_n(const PlainLaunch& L, int ngoff, const UpdArgs& UA) {
+  return L.nbr != nullptr ? launch_sweeps<NSM, true>(L, ngoff, UA) : launch_sweeps<NSM, false>(L, ngoff, UA);
+}
+
 hipError_t plain_stage(const PlainLaunch& L, int ngoff, double c1, double c2, double c3, int final_stage) {
   hipError_t e;
   const Ext E = region_ext(L, ngoff);
@@ -1236,11 +1243,9 @@ hipError_t plain_stage(const PlainLaunch& L, int ngoff, double c1, double c2, do
   // buffers
   if (L.Sin == L.Sout) return hipErrorInvalidValue;
   const UpdArgs UA{L.U0, L.Sout, L.div, L.dtp, c1, c2, c3, final_stage};
-  if (L.nbr != nullptr) {  // the neighbour table is 3D
-    if (L.P.ndim != 3) return hipErrorInvalidValue;
-    return L.P.ns == 0 ? launch_sweeps<0, true>(L, ngoff, UA) : launch_sweeps<8, true>(L, ngoff, UA);
-  }
-  return L.P.ns == 0 ? launch_sweeps<0, false>(L, ngoff, UA) : launch_sweeps<8, false>(L, ngoff, UA);
+  if (L.nbr != nullptr && L.P.ndim != 3) return hipErrorInvalidValue;  // the neighbour table is 3D
+  if (L.P.ns == 0) return launch_sweeps_n<0>(L, ngoff, UA);
+  return L.P.ns <= 4 ? launch_sweeps_n<4>(L, ngoff, UA) : launch_sweeps_n<8>(L, ngoff, UA);
 }
 
 // band: SHOK is computed over interior +/- band (the reference uses

@@ -463,3 +463,11 @@ def test_refill_3d_block_shapes(nb, n, kw):
                 blocks.append(b)
                 arrays.append(U)
     run_case(problems.Problem("refill", cfg, blocks, arrays, ug=nb), 3, f"refill {nb} x {n}")
+
+
+@pytest.mark.parametrize("nscalars", [1, 4, 5, 8])
+def test_scalar_counts(nscalars):
+    """The sweeps are built for no, up to 4 and up to 8 scalars: both sides of
+    each bound, with blocks that read their own guard cells."""
+    prob = problems.batched(nblocks=6, nguard=10, sizes=(8, 16), probs=(0.5, 0.5), shock_every=2, nscalars=nscalars)
+    run_case(prob, 2, f"{nscalars} scalars")
