@@ -686,11 +686,12 @@ __global__ void __launch_bounds__(256) k_shock(DevParams P, const BlockMeta* __r
 // leaf) from the leaves around the block, so its own guard cells need no
 // fill; the flags are still written into the block's own box.
 constexpr int SHK_T = 20;
+constexpr int SHK_GROUPS = 1536;
 constexpr int SHK_F = 5;  // staged fields: pres, sound speed, velx, vely, velz
 template <bool NB>
 __global__ void __launch_bounds__(1024) k_shock3(DevParams P, const BlockMeta* __restrict__ meta,
                                                  const int* __restrict__ blist, double* __restrict__ U, int band,
-                                                 int TW, int TH, const int64_t* __restrict__ nbr) {
+                                                 int TW, int TH, int ZL, const int64_t* __restrict__ nbr) {
   extern __shared__ double shk_lds[];
   __shared__ int64_t s_nb[27];
   const int PW = TW + 2, PS = PW * (TH + 2);
@@ -705,8 +706,10 @@ __global__ void __launch_bounds__(1024) k_shock3(DevParams P, const BlockMeta* _
     __syncthreads();
   }
   const int ex = L1.hi[0] - L1.lo[0] + 1;
-  const int ntx = (ex + TW - 1) / TW;
-  const int x0 = L1.lo[0] + (int)(blockIdx.x % ntx) * TW, y0 = L1.lo[1] + (int)(blockIdx.x / ntx) * TH;
+  const int ntx = (ex + TW - 1) / TW, nty = (L1.hi[1] - L1.lo[1] + TH) / TH;
+  const int tz = (int)blockIdx.x / (ntx * nty), txy = (int)blockIdx.x % (ntx * nty);
+  const int x0 = L1.lo[0] + txy % ntx * TW, y0 = L1.lo[1] + txy / ntx * TH;
+  const int k0 = L1.lo[2] + tz * ZL, k1 = min(k0 + ZL - 1, L1.hi[2]);  // the planes this workgroup writes
   const int tid = threadIdx.x;
   const int i = x0 + tid % TW, j = y0 + tid / TW;
   const bool own = tid < TW * TH && i <= L1.hi[0] && j <= L1.hi[1];
@@ -734,8 +737,9 @@ __global__ void __launch_bounds__(1024) k_shock3(DevParams P, const BlockMeta* _
       sv[(2 * 3 + s) * PS + u] = vz;
     }
   };
-  load(L1.lo[2]);
-  for (int k = L1.lo[2]; k <= L1.hi[2]; k++) {
+  if (k0 > L1.lo[2]) load(k0 - 1);
+  load(k0);
+  for (int k = k0; k <= k1; k++) {
     load(k + 1);
     __syncthreads();
     if (own) {
@@ -1259,15 +1263,25 @@ hipError_t plain_shock_detect(const PlainLaunch& L, double* U, double* scratch, 
     const int e1 = n[0] + 2 * band + 2, e2 = n[1] + 2 * band + 2;
     const int tw = e1 < SHK_T ? e1 : SHK_T, th = e2 < SHK_T ? e2 : SHK_T;
     const int tiles = ((e1 + tw - 1) / tw) * ((e2 + th - 1) / th);
+    // The march over z is a chain of plane loads, so columns are cut until
+    // the launch has SHK_GROUPS workgroups (twice what the chip holds), in
+    // segments of at least 3 planes; each loads 2 planes more than it writes.
+    // Per step with whole columns and cut: 64 blocks of 16^3 318 -> 284 us,
+    // 8 of 32^3 414 -> 320 us, 18 of 18 x 25 x 13 with the hybrid switch 249
+    // -> 204 us, 576 of 16^3 unchanged (768, 1536 and 2560 groups are alike).
+    const int e3 = n[2] + 2 * band + 2;
+    const int cols = tiles * L.nblk;
+    const int segs = std::max(1, std::min((SHK_GROUPS + cols - 1) / cols, e3 / 3));
+    const int zl = (e3 + segs - 1) / segs, nseg = (e3 + zl - 1) / zl;
     const int threads = (tw * th + 63) / 64 * 64;
     const size_t lds = sizeof(double) * 3 * SHK_F * (tw + 2) * (th + 2);
     if (L.prof) L.prof->begin(L.stream, "k_shock", 8.0 * nc1 * 7, nc1 * 6 + nc0 * 70);
     if (nbr)
-      hipLaunchKernelGGL(k_shock3<true>, dim3(tiles, L.nblk), dim3(threads), lds, L.stream, L.P, L.meta, L.blist, U,
-                         band, tw, th, nbr);
+      hipLaunchKernelGGL(k_shock3<true>, dim3(tiles * nseg, L.nblk), dim3(threads), lds, L.stream, L.P, L.meta,
+                         L.blist, U, band, tw, th, zl, nbr);
     else
-      hipLaunchKernelGGL(k_shock3<false>, dim3(tiles, L.nblk), dim3(threads), lds, L.stream, L.P, L.meta, L.blist, U,
-                         band, tw, th, nbr);
+      hipLaunchKernelGGL(k_shock3<false>, dim3(tiles * nseg, L.nblk), dim3(threads), lds, L.stream, L.P, L.meta,
+                         L.blist, U, band, tw, th, zl, nbr);
     if (L.prof) L.prof->end(L.stream);
     return hipGetLastError();
   }
