@@ -371,6 +371,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) k_
 
     for (int k = I.z0 - 1; k <= I.z1 + 1; k++) {
       const bool xyk = (k >= I.z0) && (k <= I.z1);
+      // a z boundary face belongs to the item holding the interior cell beside it
+      const bool zown = k == g ? k <= I.z1 : k == g + m.nz && k > I.z0;
       // ---- P1: advance the z window to k-2..k+2, stage plane k
       if (col) {
         const int64_t c = cell_at(m, nbt, g, ci, cj, k + 2);
@@ -533,7 +535,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) k_
                 shk = face_in_shock(A.U0, m, hi - sz, hi);
               }
               hydro_face<2, RIEMANN>(rp, Ls, Rs, cl, cr, Hz, A.err, shk);
-              if (regs && colin && (k == g || k == g + m.nz)) {
+              if (regs && colin && zown) {
                 const int64_t tot = (int64_t)m.nx * m.ny * (m.nz + 1);
                 const int64_t o = m.bbase + (ci - g) + (int64_t)m.nx * ((cj - g) + (int64_t)m.ny * (k - g));
                 reg_add_n<F_NUM>(A.fb[2], o, tot, 0, F_NUM, A.weight, A.add_flux, Hz);
@@ -695,7 +697,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) k_
                 else Hs[j] = xr[j] * Hz[F_MASS];
               }
             }
-            if (regs && colin && (k == g || k == g + m.nz)) {
+            if (regs && colin && zown) {
               const int64_t tot = (int64_t)m.nx * m.ny * (m.nz + 1);
               const int64_t o = m.bbase + (ci - g) + (int64_t)m.nx * ((cj - g) + (int64_t)m.ny * (k - g));
               reg_add_n<CH>(A.fb[2], o, tot, F_NUM + c0, nc, A.weight, A.add_flux, Hs);

@@ -19,7 +19,9 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <functional>
 #include <map>
+#include <queue>
 #include <set>
 #include <string>
 #include <tuple>
@@ -665,6 +667,45 @@ void partial_boxes(const spark_batch* b, int blk, int e, std::vector<Box>& out) 
   spark::sector_boxes(m.nx, m.ny, m.nz, b->p.nguard, e, b->amr_local[blk], out);
 }
 
+// Length of the z segments the column items of a stage are cut into.  A
+// workgroup marches an item level by level, two levels more than it updates
+// (the reconstruction below and the flux above), so few or unequal columns
+// leave workgroups idle, and cutting them costs those two levels per segment.
+// The length with the shortest list schedule over the launch's `slots`
+// workgroups wins, the whole column unless cutting gains 3 %.
+int z_segment(const std::vector<std::vector<spark::FusedItem>>& q, int slots) {
+  int longest = 1;
+  for (const auto& v : q)
+    for (const auto& it : v) longest = std::max(longest, it.z1 - it.z0 + 1);
+  int pick = longest;
+  double best = 0.;
+  for (int len : {longest, 24, 16, 12, 10, 8, 7, 6, 5, 4, 3}) {
+    if (len > longest) continue;
+    std::priority_queue<double, std::vector<double>, std::greater<double>> busy;
+    double end = 0.;
+    for (const auto& v : q)
+      for (const auto& it : v) {
+        const int n = it.z1 - it.z0 + 1, parts = (n + len - 1) / len, seg = (n + parts - 1) / parts;
+        // a level's time: its barriers and its columns' tasks
+        const double t = (seg + 2) * (1. + it.tx * it.ty / 64.);
+        for (int p = 0; p < parts; p++) {
+          double at = 0.;
+          if ((int)busy.size() == slots) {
+            at = busy.top();
+            busy.pop();
+          }
+          busy.push(at + t);
+          end = std::max(end, at + t);
+        }
+      }
+    if (len == longest || end < (pick == longest ? 0.97 : 1.) * best) {
+      best = end;
+      pick = len;
+    }
+  }
+  return pick;
+}
+
 // build the per-XCD queues of one stage from the chosen tiles.  A block's
 // items stay in one queue; blocks go to the least-loaded queue, largest first.
 // force_ngoff >= 0 (tuning): every block over that region.
@@ -726,6 +767,24 @@ int build_stage_plan(spark_batch* b, int stage, const std::vector<int>* only_blo
     if (tt == b->tiles.end()) return fail(SPARK_ERR_STATE, "no tile chosen for class %d ngoff %d", key.first, ngoff);
     box_items(id, region_box(m, b->p.nguard, ngoff), tt->second.first, tt->second.second, q[qi]);
   }
+  size_t lds = 0;
+  for (const auto& v : q)
+    for (const auto& it : v) lds = std::max(lds, fused_lds(b, it.tx, it.ty));
+  b->stage_lds[stage - 1] = lds;
+  b->stage_grid[stage - 1] = fused_grid_for(b, b->stage_lds[stage - 1]);
+  const int len = z_segment(q, b->stage_grid[stage - 1]);
+  for (auto& v : q) {
+    std::vector<spark::FusedItem> cut;
+    for (const auto& it : v) {
+      const int n = it.z1 - it.z0 + 1, parts = (n + len - 1) / len, seg = (n + parts - 1) / parts;
+      for (int z = it.z0; z <= it.z1; z += seg) {
+        cut.push_back(it);
+        cut.back().z0 = z;
+        cut.back().z1 = std::min(z + seg - 1, it.z1);
+      }
+    }
+    v.swap(cut);
+  }
   auto& pl = b->plan[stage - 1];
   pl.items.clear();
   int qoff[spark::FUSED_XCDS], qlen[spark::FUSED_XCDS];
@@ -741,10 +800,6 @@ int build_stage_plan(spark_batch* b, int stage, const std::vector<int>* only_blo
   HIPCHK(hipMemcpy(pl.items_d, pl.items.data(), sizeof(spark::FusedItem) * pl.items.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(pl.qoff_d, qoff, sizeof(qoff), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(pl.qlen_d, qlen, sizeof(qlen), hipMemcpyHostToDevice));
-  size_t lds = 0;
-  for (const auto& it : pl.items) lds = std::max(lds, fused_lds(b, it.tx, it.ty));
-  b->stage_lds[stage - 1] = lds;
-  b->stage_grid[stage - 1] = fused_grid_for(b, b->stage_lds[stage - 1]);
   return SPARK_OK;
 }
 

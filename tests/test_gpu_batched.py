@@ -341,3 +341,35 @@ def test_plain_short_quotients_equal_ieee_divides():
     for x, y in zip(interiors(prob, res[0][1]), interiors(prob, res[1][1])):
         assert np.array_equal(x, y, equal_nan=True)
         assert np.isfinite(x[..., : capi.SPARK_NPROP + 4]).all()
+
+
+@pytest.mark.parametrize("n,nscalars", [(8, 0), (11, 2)])
+def test_fp32_columns_cut_along_z_equal_whole_columns(n, nscalars):
+    """A batch of few blocks runs its columns in z segments, one of many blocks
+    in longer ones: the same block must come out bit for bit the same, its
+    flux registers included (a face on a segment's end is accumulated once)."""
+    one = problems.batched(nblocks=1, nguard=10, sizes=(n,), probs=(1.0,), shock_every=1, nscalars=nscalars)
+    res = []
+    for copies in (1, 40, 300):
+        prob = problems.Problem("copies", dict(one.cfg, flux_correct=1, form="fp32_flux"), list(one.blocks) * copies,
+                                [one.arrays[0]] * copies)
+        b = capi.Batch(prob.cfg, prob.blocks)
+        try:
+            b.pack(prob.arrays)
+            dt = b.compute_dt()[0]
+            b.hydro_step(dt)
+            out = [a.copy() for a in prob.arrays]
+            b.unpack(out, interior_only=True)
+            regs = [[np.zeros((5 + nscalars, n + (d == 2), n + (d == 1), n + (d == 0))) for _ in range(copies)]
+                    for d in range(3)]
+            b.get_flux_registers(*regs)
+        finally:
+            b.close()
+        res.append((dt, out, regs))
+    for dt, out, regs in res:
+        assert dt == res[0][0]
+        for k in (0, len(out) - 1):
+            assert np.array_equal(out[k], res[0][1][0])
+            for d in range(3):
+                assert np.array_equal(regs[d][k], res[0][2][d][0])
+                assert np.any(regs[d][k] != 0.0)
