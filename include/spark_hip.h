@@ -35,10 +35,11 @@ extern "C" {
 
 enum spark_recon { SPARK_RECON_WENO5 = 0, SPARK_RECON_MP5 = 1, SPARK_RECON_PLM = 2, SPARK_RECON_FOG = 3 };
 enum spark_riemann { SPARK_RIEMANN_HLLC = 0, SPARK_RIEMANN_HLL = 1 };
-/* plain FP64 form (one launch per kernel per stage, materialised face
- * fluxes); batched form (one fused persistent launch per stage over blocks
- * of any size) with FP32 reconstruction/Riemann arithmetic and FP64
- * accumulation, or in FP64 throughout */
+/* plain FP64 form (directional sweeps, one launch per sweep, stage and block
+ * shape); FP32-flux form (one fused persistent launch per stage over blocks
+ * of any size, FP32 reconstruction/Riemann arithmetic and FP64
+ * accumulation); batched FP64 form (the plain form's sweeps; its stage entry
+ * points read same-level halos as the FP32-flux form's do) */
 enum spark_form { SPARK_FORM_PLAIN_FP64 = 0, SPARK_FORM_FP32_FLUX = 1, SPARK_FORM_BATCHED_FP64 = 2 };
 /* guard policy: telescoping stages over guard cells filled once per step
  * (the reference's own scheme, Spark/Hydro.ini:19,37), or refilling the
@@ -296,7 +297,8 @@ int spark_profile_read(spark_batch* b, spark_kernel_stat* stats, int max, int* n
 #define SPARK_OPT_AUTOTUNE 2
 #define SPARK_OPT_SAME_LEVEL_HALOS 3
 int spark_set_option(spark_batch* b, int option, int value);
-/* Tiles chosen by the batched form: rows of (nx, ny, nz, ngoff, tx, ty). */
+/* Tiles chosen by the batched forms: rows of (nx, ny, nz, ngoff, tx, ty); the
+ * batched FP64 form runs whole regions, (tx, ty) their cross-sections. */
 int spark_batched_tiles(spark_batch* b, int* rows, int max_rows, int* nrows);
 
 int spark_synchronize(spark_batch* b);
