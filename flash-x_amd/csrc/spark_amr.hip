@@ -9,6 +9,7 @@
 // the leaf under any cell of any level is one table read away.
 #include <hip/hip_runtime.h>
 
+#include "spark_batched.hpp"
 #include "spark_launch.hpp"
 
 namespace spark {
@@ -220,6 +221,44 @@ __global__ void __launch_bounds__(256) k_amr_fill(DevParams P, const BlockMeta* 
   }
 }
 
+// Guard sectors that a block reads from the leaves around it, copied into its
+// own box: cells of depth <= depth in the sectors of cmask, from where cell_at
+// finds them (a leaf's interior, or a sector that leaf computes, which is in
+// no cmask of its own, so no cell is read and written).  Bound by memory, and
+// by the 8-byte islands of the x layers as the guard fill is.
+__global__ void __launch_bounds__(256) k_halo_copy(DevParams P, const BlockMeta* __restrict__ meta,
+                                                   const int64_t* __restrict__ nbr, AmrGrid G, double* __restrict__ U,
+                                                   VarList vars, int depth, const uint32_t* __restrict__ cmask) {
+  const int bid = (int)blockIdx.y;
+  const uint32_t mk = cmask[bid];
+  if (mk == 0) return;
+  const BlockMeta m = meta[bid];
+  const int n = G.n, g = P.ng, ext = n + 2 * depth, total = ext * ext * ext;
+  const int64_t* nbt = nbr + (int64_t)bid * 27;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
+    const int loc[3] = {g - depth + t % ext, g - depth + (t / ext) % ext, g - depth + t / (ext * ext)};
+    int sec = 13;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int sd = d == 0 ? 1 : d == 1 ? 3 : 9;
+      sec += loc[d] < g ? -sd : loc[d] >= g + n ? sd : 0;
+    }
+    if (!((mk >> sec) & 1u)) continue;
+    const int64_t src = cell_at(m, nbt, g, loc[0], loc[1], loc[2]);
+    const int64_t dst = m.base + acix(m.PX, m.NX, loc[0], loc[1], loc[2]);
+    // loads of a chunk before its stores (see k_amr_fill)
+    constexpr int CHV = 8;
+    for (int q0 = 0; q0 < vars.n; q0 += CHV) {
+      double val[CHV];
+#pragma unroll
+      for (int u = 0; u < CHV; u++) val[u] = U[src + vars.v[q0 + u < vars.n ? q0 + u : vars.n - 1] * m.cstride];
+#pragma unroll
+      for (int u = 0; u < CHV; u++)
+        if (q0 + u < vars.n) U[dst + vars.v[q0 + u] * m.cstride] = val[u];
+    }
+  }
+}
+
 // Flux-register exchange for direction dir: on each boundary face of a
 // block whose neighbour across is a finer leaf, the correction is the mean
 // of the 4 fine faces (red_f = 0.25 for flux densities,
@@ -300,6 +339,18 @@ hipError_t amr_fill(const PlainLaunch& L, const AmrGrid& G, double* U, const Var
   if (L.prof) L.prof->begin(L.stream, "k_amr_fill", 16.0 * L.nblk * (double)(box - nin) * vars.n, 0.0);
   hipLaunchKernelGGL(k_amr_fill, dim3(grid_x(box, 512), L.nblk), dim3(256), 0, L.stream, L.P, L.meta, L.blist, G, U,
                      vars, depth, smask, keep);
+  if (L.prof) L.prof->end(L.stream);
+  return hipGetLastError();
+}
+
+hipError_t amr_halo_copy(const PlainLaunch& L, const AmrGrid& G, double* U, const VarList& vars, int depth,
+                         const uint32_t* cmask) {
+  if (depth < 1) return hipSuccess;
+  const int ext = G.n + 2 * depth;
+  const int box = ext * ext * ext;
+  if (L.prof) L.prof->begin(L.stream, "k_halo_copy", 16.0 * L.nblk * (double)(box - G.n * G.n * G.n) * vars.n, 0.0);
+  hipLaunchKernelGGL(k_halo_copy, dim3(grid_x(box, 512), L.nblk), dim3(256), 0, L.stream, L.P, L.meta, L.nbr, G, U, vars,
+                     depth, cmask);
   if (L.prof) L.prof->end(L.stream);
   return hipGetLastError();
 }

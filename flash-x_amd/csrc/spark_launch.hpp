@@ -133,6 +133,10 @@ enum { AMR_BC_OUTFLOW = 0, AMR_BC_PERIODIC = 1, AMR_BC_REFLECT = 2 };
 // only to `keep` layers
 hipError_t amr_fill(const PlainLaunch& L, const AmrGrid& G, double* U, const VarList& vars, int depth,
                     const uint32_t* smask = nullptr, int keep = 0);
+// the guard sectors of cmask (per block) to `depth`, copied through the
+// neighbour table L.nbr into the blocks' own boxes
+hipError_t amr_halo_copy(const PlainLaunch& L, const AmrGrid& G, double* U, const VarList& vars, int depth,
+                         const uint32_t* cmask);
 hipError_t amr_flux_exchange(const PlainLaunch& L, const AmrGrid& G, double* const fb[3], double* const fc[3]);
 hipError_t plain_aos_to_soa(hipStream_t st, const BlockMeta* meta, int nblk, int maxcells, const double* aos,
                             const int64_t* aos_off, int nunk, const int* var_index, int nvar, double* U);

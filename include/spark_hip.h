@@ -140,9 +140,28 @@ int spark_pack(spark_batch* b, const double* const* unk_blocks);
 int spark_pack_noalloc(spark_batch* b, const double* const* unk_blocks);
 /* Device -> host unk blocks; interior_only mirrors updateState
  * (Spark/Hydro_funcs.F90-mc:573-574) and writes only the interior cells;
- * unk slots outside the variable map keep their host values.  which = 0: solution, 1: the stage
- * state (hy_starState) written by the last stage run before a step's final
- * stage. */
+ * unk slots outside the variable map keep their host values.  which = 0:
+ * solution, 1: the stage state (hy_starState) written by the last stage run
+ * before a step's final stage.  Guard cells (interior_only = 0): spark_hydro_step
+ * and spark_advance write no guard cell of the new solution (updateState copies
+ * the interior), so after them the guards of the solution hold the guard fill
+ * at the start of the last step, as the reference's unk does, and those of the
+ * stage state what the last stage before the final one computed there, or the
+ * refill after it:
+ *   plain form                   solution: the layers the first stage reaches
+ *                                (refill: nstencil layers); stage state: the
+ *                                layers that stage covers (refill: nstencil)
+ *   batched forms, 3D refill     solution: one layer, two with the hybrid
+ *                                solver; stage state: none
+ *   batched forms, hierarchy     solution: the guard sectors (face, edge or
+ *                                corner regions of the guard band) with no
+ *                                leaf of the block's own level across them,
+ *                                and of blocks with such sectors the first
+ *                                layer of the others (every layer with the
+ *                                hybrid solver); stage state: those sectors
+ *   batched forms, otherwise     as the plain form
+ * Other guard cells keep what they held.  spark_fill_guardcells fills all of
+ * the solution's from its present interior. */
 int spark_unpack(spark_batch* b, double* const* unk_blocks, int interior_only, int which);
 
 /* Declare the batch a uniform nbx x nby x nbz block grid (blocks numbered
@@ -162,11 +181,14 @@ int spark_set_uniform_grid(spark_batch* b, int nbx, int nby, int nbz);
  * Enables the device guard fill over levels (same-level copy, the mean of 8
  * cells of a finer leaf, limited linear prolongation from a coarser leaf)
  * and, with flux_correct, the device flux-register exchange after every
- * step.  In the batched forms a leaf whose 26 neighbours are leaves of its
- * own level reads its halo from them and updates only its interior in every
- * stage (the values telescoping would give; such a leaf's own guard cells
- * are not filled by the step: spark_fill_guardcells fills them on request);
- * with flux_correct the
+ * step.  In spark_hydro_step and spark_advance, and in the batched forms'
+ * stage entry points, a leaf reads a guard sector with a leaf of its own level
+ * across it from that leaf, and an edge or corner sector beside a leaf of its
+ * level that computes it from that leaf's guard cells, and computes only its
+ * interior and the other sectors (the values telescoping would give;
+ * spark_unpack says which guard cells are left in its own box).  The plain
+ * form's stage entry points telescope over the block's own guard cells:
+ * spark_fill_guardcells goes before them.  With flux_correct the
  * FP32-flux form corrects only the cells on faces toward a finer leaf (the
  * correction is zero elsewhere; the FP64 forms still pass those cells
  * through the reference's conserved/primitive round trip).
@@ -188,8 +210,8 @@ int spark_fill_guardcells(spark_batch* b);
  * Driver/DriverMain/Driver_computeDt.F90:306. */
 int spark_compute_dt(spark_batch* b, double* dt, int minloc[5]);
 
-/* One full RK step of every block: the guard fill when a uniform grid was
- * declared (Spark/Hydro.F90-mc:106), shockDetect, saveState, the stages,
+/* One full RK step of every block: the guard fill when a uniform grid or a
+ * hierarchy was declared (Spark/Hydro.F90-mc:106), shockDetect, saveState, the stages,
  * updateState; flux registers when flux_correct.
  * Replaces: Hydro(timeEndAdv, dt, dtOld, sweepOrder),
  * Hydro_interface.F90:61-66 / Spark/Hydro.F90-mc:24-202. */
@@ -204,7 +226,7 @@ int spark_stage(spark_batch* b, int stage, double dt, int ngoff);
 int spark_step_end(spark_batch* b);
 
 /* nsteps device-resident steps: dt (CFL, on the device) -> guard fill (if a
- * uniform grid was declared) -> step.  dts (optional, nsteps) receives the
+ * grid was declared; only the cells a step reads before the last one) -> step.  dts (optional, nsteps) receives the
  * dt used at each step.  No host synchronisation between steps.
  * Replaces: the Hydro / Driver_computeDt pair of the step loop,
  * Driver/DriverMain/Unsplit/Driver_evolveAll.F90:136-275. */
@@ -287,11 +309,10 @@ int spark_profile_read(spark_batch* b, spark_kernel_stat* stats, int max, int* n
  * into a hipGraph and replays it.  SPARK_OPT_AUTOTUNE (default 1): the
  * batched FP32-flux form times candidate tile shapes per block shape and
  * stage region on the first step and keeps the fastest.
- * SPARK_OPT_SAME_LEVEL_HALOS (default 1): on a block hierarchy the batched
- * forms let a leaf read each guard sector (face, edge or corner region of
- * its guard band) that has a leaf of its own level across from that leaf,
- * and telescope only over the others; 0 makes every leaf telescope over
- * all its guard cells (the same values, more work).  No counterpart in the
+ * SPARK_OPT_SAME_LEVEL_HALOS (default 1): on a block hierarchy a leaf reads
+ * guard sectors from leaves of its own level (spark_set_amr_grid) and
+ * telescopes only over the others; 0 makes every leaf telescope over all its
+ * guard cells (the same values, more work).  No counterpart in the
  * reference. */
 #define SPARK_OPT_GRAPH 1
 #define SPARK_OPT_AUTOTUNE 2
