@@ -182,12 +182,11 @@ struct spark_batch {
   bool autotune = true;
   int* tune_err = nullptr;    // Riemann-error counter of tuning launches
   double* tune_dt = nullptr;  // dt = 0 of tuning launches (the batch's dt stays untouched)
-  // graphs of one device-resident step (dt, guard fill, stages): of a run's
-  // steps and of the step a call ends with (step_differs)
+  // graph of one device-resident step (dt, guard fill, stages)
   bool use_graph = true;
   int* hist_slot = nullptr;
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t gexec = nullptr;
   int last_stage = 3;
   double coeff[3][3];
   int limits_array[3];
@@ -999,12 +998,10 @@ int plain_groups_build(spark_batch* b) {
 }
 
 void drop_graph(spark_batch* b) {
-  for (int q = 0; q < 2; q++) {
-    if (b->gexec[q]) (void)hipGraphExecDestroy(b->gexec[q]);
-    if (b->graph[q]) (void)hipGraphDestroy(b->graph[q]);
-    b->gexec[q] = nullptr;
-    b->graph[q] = nullptr;
-  }
+  if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+  if (b->graph) (void)hipGraphDestroy(b->graph);
+  b->gexec = nullptr;
+  b->graph = nullptr;
 }
 
 }  // namespace
@@ -1488,24 +1485,6 @@ static int one_step(spark_batch* b, bool last) {
   return rc ? rc : run_step(b, last);
 }
 
-// capture one device-resident step; every parameter of it lives on the
-// device (dt, the dt-history slot, the queue heads), so replays chain
-static int capture_step(spark_batch* b, bool last) {
-  if (b->gexec[last]) return SPARK_OK;
-  HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-  const int rc = one_step(b, last);
-  hipGraph_t gr = nullptr;
-  hipError_t e = hipStreamEndCapture(g_stream, &gr);
-  if (rc) {
-    if (gr) (void)hipGraphDestroy(gr);
-    return rc;
-  }
-  if (e != hipSuccess) return fail(SPARK_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-  b->graph[last] = gr;
-  HIPCHK(hipGraphInstantiate(&b->gexec[last], gr, nullptr, nullptr, 0));
-  return SPARK_OK;
-}
-
 int spark_advance(spark_batch* b, int nsteps, double* dts) {
   if (!b) return fail(SPARK_ERR_ARG, "spark_advance: null batch");
   if (nsteps < 0) return fail(SPARK_ERR_ARG, "nsteps = %d", nsteps);
@@ -1522,22 +1501,35 @@ int spark_advance(spark_batch* b, int nsteps, double* dts) {
   if (b->fused && !b->planned && (rc = fused_plan(b))) return rc;
   HIPCHK(spark::plain_set_int(g_stream, b->hist_slot, 0));
   const bool graph = b->use_graph && !b->prof.on && nsteps > 0;
+  // replayed steps; the one the call ends with is launched as it is where it
+  // differs (behind the replays, and a graph of its own costs half a
+  // millisecond once)
   const bool differs = step_differs(b);
-  if (graph && !b->gexec[0] && !b->gexec[1] && b->amr && b->p.flux_correct && !b->fc_clean) {
+  const int replays = graph ? nsteps - (differs ? 1 : 0) : 0;
+  if (graph && b->gexec == nullptr && b->amr && b->p.flux_correct && !b->fc_clean) {
     // zero the corrections outside the graph so that the captured exchange
     // visits only the blocks with a finer face
     for (int d = 0; d < 3; d++) HIPCHK(hipMemsetAsync(b->fc[d], 0, sizeof(double) * b->bpool, g_stream));
     b->fc_clean = true;
   }
-  if (graph && (nsteps > 1 || !differs) && (rc = capture_step(b, false))) return rc;
-  if (graph && differs && (rc = capture_step(b, true))) return rc;
-  for (int s = 0; s < nsteps; s++) {
-    const bool last = differs && s == nsteps - 1;
-    if (graph) {
-      HIPCHK(hipGraphLaunch(b->gexec[last], g_stream));
-    } else if ((rc = one_step(b, last))) {
+  if (replays > 0 && b->gexec == nullptr) {
+    // capture one device-resident step; every parameter of it lives on the
+    // device (dt, the dt-history slot, the queue heads), so replays chain
+    HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
+    rc = one_step(b, false);
+    hipGraph_t gr = nullptr;
+    hipError_t e = hipStreamEndCapture(g_stream, &gr);
+    if (rc) {
+      if (gr) (void)hipGraphDestroy(gr);
       return rc;
     }
+    if (e != hipSuccess) return fail(SPARK_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
+    b->graph = gr;
+    HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
+  }
+  for (int s = 0; s < nsteps; s++) {
+    if (s < replays) HIPCHK(hipGraphLaunch(b->gexec, g_stream));
+    else if ((rc = one_step(b, differs && s == nsteps - 1))) return rc;
   }
   if (dts && nsteps > 0) {
     HIPCHK(hipMemcpyAsync(dts, b->dt_hist, sizeof(double) * nsteps, hipMemcpyDeviceToHost, g_stream));
