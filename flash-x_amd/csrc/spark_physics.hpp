@@ -135,15 +135,18 @@ __device__ __forceinline__ double rcp_in_range(double b) {
 // weno5<double> with the short quotients, bit for bit the expressions above.
 // A third of the reconstruction's instructions were the five IEEE divides of
 // the weights; a wave takes the short ones unless a lane is out of their
-// range.  With beta1 + beta3 < 2^900 every beta is small (two small
-// differences of a 3-point stencil make its values equal to rounding, so
-// beta2 cannot be large alone), the ratios tau / (beta + 1e-36) stay under
-// 2^1020 and the weight sums between 1 and 2^1021: no quotient that counts
-// would be scaled (a tau so small that its quotient underflows adds nothing
-// to 1).  Otherwise, NaN and infinities included, the wave divides in full.
-// The products by 2, 4 and 0.25 are exact (0.25 s^2 underflows only where the
-// 1e-36 swamps it), so fusing them with the addition that follows rounds the
-// same: 8 fewer instructions.  Sweeps of 576 blocks of 16^3 with 8 scalars,
+// range: u0^2 + beta1 + beta3 < 2^900.  Then |u0| < 2^450, and t1, s1 (t3, s3)
+// below 2^452 leave the other values of the stencil within 2^453 of it
+// (2 (u0 - um1) = s1 - t1; what rounding hides of a slope is a few ulps of
+// 2^453), so beta2 < 2^910 (without the bound on u0, values an ulp apart above
+// 2^560 have beta1 = beta3 = 0 beside an infinite beta2).  The ratios
+// tau / (beta + 1e-36) stay under 2^1020 and the weight sums between 1 and
+// 2^1021: no quotient that counts would be scaled (a tau so small that its
+// quotient underflows adds nothing to 1).  The products by 2, 4 and 0.25 are
+// exact (0.25 s^2 underflows only where the 1e-36 swamps it), so fusing them
+// with the addition that follows rounds the same: 8 fewer instructions.
+// Otherwise, NaN and infinities included, the wave takes the expressions above
+// as they stand.  Sweeps of 576 blocks of 16^3 with 8 scalars,
 // telescoping: x 2.87 -> 2.65, y 3.39 -> 3.29, z 4.56 -> 4.44 ms per step.
 // (One range test after all variables, and the whole reconstruction again
 // where it fails, spills and measured 2.79 / 3.38 / 4.55.)
@@ -157,17 +160,22 @@ __device__ __forceinline__ void weno5_short(double um2, double um1, double u0, d
   const double s1 = __builtin_fma(-4., um1, um2) + u03;
   const double s2 = um1 - up1;
   const double s3 = __builtin_fma(-4., up1, u03) + up2;
-  const double b1 = __builtin_fma(0.25, s1 * s1, n13o12 * (t1 * t1));
-  const double b2 = __builtin_fma(0.25, s2 * s2, n13o12 * (t2 * t2));
-  const double b3 = __builtin_fma(0.25, s3 * s3, n13o12 * (t3 * t3));
-  const double tau = __builtin_fabs(b1 - b3);
-  const bool in_range = __ballot(!(b1 + b3 < 0x1p900)) == 0;
+  double b1 = __builtin_fma(0.25, s1 * s1, n13o12 * (t1 * t1));
+  double b2 = __builtin_fma(0.25, s2 * s2, n13o12 * (t2 * t2));
+  double b3 = __builtin_fma(0.25, s3 * s3, n13o12 * (t3 * t3));
+  const bool in_range = __ballot(!(__builtin_fma(u0, u0, b1) + b3 < 0x1p900)) == 0;
   double r1, r2, r3;
   if (in_range) {
+    const double tau = __builtin_fabs(b1 - b3);
     r1 = div_in_range(tau, b1 + eps);
     r2 = div_in_range(tau, b2 + eps);
     r3 = div_in_range(tau, b3 + eps);
   } else {
+    auto beta = [&](double t, double s) { return n13o12 * (t * t) + 0.25 * (s * s); };
+    b1 = beta(um2 - 2. * um1 + u0, um2 - 4. * um1 + 3. * u0);
+    b2 = beta(um1 - 2. * u0 + up1, um1 - up1);
+    b3 = beta(u0 - 2. * up1 + up2, 3. * u0 - 4. * up1 + up2);
+    const double tau = __builtin_fabs(b1 - b3);
     r1 = tau / (b1 + eps);
     r2 = tau / (b2 + eps);
     r3 = tau / (b3 + eps);
