@@ -83,11 +83,10 @@ struct spark_batch {
   std::vector<BlockMeta> meta_h;
   BlockMeta* meta_d = nullptr;
   std::vector<ShapeClass> classes;
-  int64_t pool = 0, opool = 0, dpool = 0, bpool = 0;  // sizes in doubles
+  int64_t pool = 0, opool = 0, bpool = 0;  // sizes in doubles
   double* U = nullptr;
   double* S = nullptr;
   double* flat = nullptr;
-  double* div = nullptr;  // plain form: the sweeps' divergence terms per cell
   double* fb[3] = {nullptr, nullptr, nullptr};
   double* dtp = nullptr;
   long long* loc = nullptr;
@@ -229,7 +228,7 @@ PlainLaunch make_launch(spark_batch* b, const ShapeClass& c) {
   L.Sin = b->S;
   L.Sout = b->S;
   L.flat = b->flat;
-  L.div = b->div;
+  L.div = nullptr;
   for (int d = 0; d < 3; d++) L.fb[d] = b->p.flux_correct ? b->fb[d] : nullptr;
   L.weight = 0.;
   L.add_flux = 0;
@@ -482,6 +481,16 @@ double* stage_out(spark_batch* b, int stage) {
   return stage == 1 ? b->S : b->S2;
 }
 
+// where the sweeps of a stage keep their divergence terms: the stage's own
+// output, and in the last stage, which writes the solution its update reads,
+// the buffer that stage does not use (S is not read again after stage 2 of RK3,
+// RK2 has no stage 2 buffer).  A pool of their own (5 + N_s fields) would take a
+// fifth more memory than the state.
+double* stage_div(spark_batch* b, int stage) {
+  if (stage != b->last_stage) return stage_out(b, stage);
+  return b->last_stage == 3 ? b->S : b->S2;
+}
+
 int stage_ngoff(const spark_batch* b, int stage) {
   return b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[stage - 1];
 }
@@ -560,6 +569,7 @@ int run_stage_groups(spark_batch* b, int stage) {
   L.add_flux = stage > 1;
   L.Sin = stage_in(b, stage);
   L.Sout = out;
+  L.div = stage_div(b, stage);
   for (const auto& g : b->groups[stage - 1]) {
     PlainLaunch G = L;
     G.blist = g.ids_d;
@@ -606,6 +616,7 @@ int run_stage(spark_batch* b, int stage, int ngoff, bool same_level) {
     L.add_flux = stage > 1;
     L.Sin = stage_in(b, stage);
     L.Sout = stage_out(b, stage);
+    L.div = stage_div(b, stage);
     if (same_level && ug_remap(b)) L.nbr = b->nbr_d;
     HIPCHK(spark::plain_stage(L, ngoff, co[0], co[1], co[2], stage == b->last_stage));
   }
@@ -684,7 +695,6 @@ void free_batch(spark_batch* b) {
   F(b->meta_d);
   for (auto& c : b->classes) F(c.ids_d);
   F(b->U); F(b->S); F(b->flat);
-  F(b->div);
   for (int d = 0; d < 3; d++) F(b->fb[d]);
   F(b->dtp); F(b->loc); F(b->dt_hist); F(b->dtparts); F(b->err);
   delete b;
@@ -1154,15 +1164,15 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
 
   const int g = p->nguard;
   const int nf = 5 + p->nscalars;
-  // rows are padded (row_pad) unless that would take the state past half of a
-  // GPU's memory
+  size_t free_bytes = 0, total_bytes = 0;
+  if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) free_bytes = 0;
   int64_t padded = 0;
   for (int i = 0; i < nblocks; i++) {
     const int NX = blocks[i].nx + 2 * g;
     padded += (int64_t)spark::row_pad(NX, g).pitch * (p->ndim > 1 ? blocks[i].ny + 2 * g : 1) *
               (p->ndim > 2 ? blocks[i].nz + 2 * g : 1);
   }
-  const bool pad_rows = padded * (3 * nvar + nf + 1) < (int64_t(128) << 30) / (int64_t)sizeof(double);
+  const bool pad_rows = spark::pad_rows(padded, 3 * nvar + 1, (int64_t)free_bytes);
   std::map<std::tuple<int, int, int>, int> cls;
   int64_t max_int = 0;
   for (int i = 0; i < nblocks; i++) {
@@ -1186,8 +1196,6 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
     b->pool += (int64_t)nvar * m.cstride;
     m.obase = b->opool + rp.lead;
     b->opool += m.cstride;
-    m.dbase = b->dpool + rp.lead;
-    b->dpool += (int64_t)nf * m.cstride;
     int64_t reg = 1;
     for (int q = 0; q < 3; q++) reg *= n[q] + (q < p->ndim ? 1 : 0);
     m.bbase = b->bpool;
@@ -1226,9 +1234,6 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   ALLOC(b->S, sizeof(double) * b->pool);
   ALLOC(b->flat, sizeof(double) * b->opool);
   ALLOC(b->S2, sizeof(double) * b->pool);
-  // the divergence terms of the sweeps (the sweeps before the last write
-  // them; 1D has no earlier sweep)
-  if (p->form != SPARK_FORM_FP32_FLUX && p->ndim > 1) ALLOC(b->div, sizeof(double) * b->dpool);
   if (p->flux_correct) {
     for (int q = 0; q < 3; q++) ALLOC(b->fb[q], sizeof(double) * b->bpool);
     for (int q = 0; q < 3; q++) ALLOC(b->fc[q], sizeof(double) * b->bpool);
@@ -1266,7 +1271,6 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   HIPCHK(hipMemsetAsync(b->S, 0, sizeof(double) * b->pool, g_stream));
   HIPCHK(hipMemsetAsync(b->flat, 0, sizeof(double) * b->opool, g_stream));
   HIPCHK(hipMemsetAsync(b->S2, 0, sizeof(double) * b->pool, g_stream));
-  if (b->div) HIPCHK(hipMemsetAsync(b->div, 0, sizeof(double) * b->dpool, g_stream));
   if (p->flux_correct)
     for (int q = 0; q < 3; q++) HIPCHK(hipMemsetAsync(b->fb[q], 0, sizeof(double) * b->bpool, g_stream));
   HIPCHK(hipMemsetAsync(b->err, 0, sizeof(int), g_stream));

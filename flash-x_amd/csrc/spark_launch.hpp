@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "spark_physics.hpp"
+#include "spark_rows.hpp"
 
 namespace spark {
 
@@ -37,23 +38,6 @@ struct Prof {
   }
 };
 
-// Rows of a block's guard-celled box in the pools: `pitch` doubles apart, the
-// box `lead` doubles into its place, so that every row's first interior cell
-// starts a 128-byte line (a 64-byte half line where full lines would cost more
-// than a third of the memory; rows stay packed where that does too).  The
-// sweeps are bound by the lines their rows touch: 16 cells of a packed 36-cell
-// row lie across two lines or three halves and share them with guard cells.
-// 576 leaves of 16^3 with 8 scalars, FP64: the sweeps over the interiors
-// fetched 2.6 and wrote 1.3 GB per stage packed, 1.4 and 1.0 GB aligned.
-struct RowPad { int pitch, lead; };
-inline RowPad row_pad(int NX, int ng) {
-  for (int a : {16, 8}) {
-    const int pitch = (NX + a - 1) / a * a;
-    if (3 * pitch <= 4 * NX) return RowPad{pitch, (a - ng % a) % a};
-  }
-  return RowPad{NX, 0};
-}
-
 // offset of cell t of a block's guard-celled box, cells counted x fastest
 // without the padding
 __device__ __forceinline__ int64_t box_cell(const BlockMeta& m, int64_t t) {
@@ -82,7 +66,7 @@ struct PlainLaunch {
   const double* Sin;      // stage input state (U at stage 1, S after)
   double* Sout;           // stage output state (U at the last stage, S before)
   double* flat;           // flattening coefficients / scratch (cell pool)
-  double* div;            // divergence terms of the sweeps so far (cell pool, 5 + ns fields)
+  double* div;            // state buffer holding the divergence terms of the sweeps so far (2D, 3D)
   double* fb[3];          // flux-register pools (nullptr when not correcting)
   double weight;          // flux-register weight of this stage
   int add_flux;           // 0: overwrite (stage 1), 1: accumulate
