@@ -11,11 +11,14 @@
 #include <algorithm>
 #include <atomic>
 #include <deque>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
+#include <utility>
+#include <vector>
 
 #include "spark_transfer.hpp"
+#include "spark_workers.hpp"
 
 namespace spark {
 namespace {
@@ -288,24 +291,13 @@ hipError_t transfer(const XferJob& j, double* const* host, bool pack, int device
     }
     if (r != hipSuccess) fail(r);
   };
-  std::vector<std::thread> threads;
-  auto guarded = [&](int w) {
+  run_workers(workers, [&](int w) {
     try {
       work(w);
     } catch (const std::exception&) {
       fail(hipErrorOutOfMemory);
     }
-  };
-  threads.reserve(workers);
-  for (int w = 1; w < workers; w++) {
-    try {
-      threads.emplace_back(guarded, w);
-    } catch (const std::system_error&) {
-      break;  // fewer threads: the others take the chunks
-    }
-  }
-  guarded(0);
-  for (auto& t : threads) t.join();
+  });
   e = (hipError_t)failed.load();
   for (Slot& s : g_staging.slot) {
     if (!s.used) continue;

@@ -8,9 +8,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <functional>
-#include <vector>
-
 #include "spark_launch.hpp"
 #include "spark_physics.hpp"
 
