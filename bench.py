@@ -214,6 +214,20 @@ NUM_CU = 256
 CLOCK_HZ = 2.4e9  # MI355X peak engine clock
 
 
+def kernel_key():
+    """Identifies the code the counters of a summary belong to: a hash of the
+    library's sources and build flags without comments and white space."""
+    import hashlib
+    import re
+    h = hashlib.sha256()
+    pkg = ROOT / "flash-x_amd"
+    for f in [pkg / "Makefile"] + sorted(p for p in (pkg / "csrc").iterdir() if p.suffix in (".hip", ".hpp", ".cpp")):
+        text = f.read_text()
+        text = re.sub(r"#.*" if f.name == "Makefile" else r"//[^\n]*|/\*(?:.|\n)*?\*/", "", text)
+        h.update(f.name.encode() + b"\0" + re.sub(r"\s+", "", text).encode() + b"\0")
+    return h.hexdigest()[:16]
+
+
 def _csv_rows(path):
     import csv
     with open(path, newline="") as f:
@@ -309,17 +323,25 @@ def summarize(args):
                      "read + write (torch.neg): " + ", ".join(f"{c} x{v:.3f}" for c, v in sorted(scale.items())) +
                      "; the runtime's blit copy of 1 GiB reads as " +
                      ", ".join(f"{c} {v / true_bytes:.3f}" for c, v in sorted(blit.items())) + " of its bytes")
+    lines.append(KEY_LINE + kernel_key())
     print("\n".join(lines))
 
 
-def read_counter_summary(workload, form):
+KEY_LINE = "# counters of the code with key "
+
+
+def read_counter_summary(workload, form, folder=ROOT / "profiles"):
     """The committed per-kernel counter table of one form of a workload
-    (written by --summarize), as {kernel: {column: value}}, or None."""
-    path = ROOT / "profiles" / f"{workload}_{form}_counters.txt"
+    (written by --summarize): (table, None) with the table as {kernel:
+    {column: value}}, or (None, why it is not used).  Counters are only used
+    beside times of the code they were taken from."""
+    path = folder / f"{workload}_{form}_counters.txt"
     if not path.exists():
-        return None
-    cols, out = None, {}
+        return None, f"no {path.name}"
+    cols, out, key = None, {}, None
     for ln in path.read_text().splitlines():
+        if ln.startswith(KEY_LINE):
+            key = ln[len(KEY_LINE):].strip()
         if ln.startswith("#") or not ln.strip():
             continue
         parts = [x.strip() for x in ln.split("|")]
@@ -327,7 +349,40 @@ def read_counter_summary(workload, form):
             cols = parts
             continue
         out[parts[0]] = {c: (None if v == "-" else float(v)) for c, v in zip(cols[1:], parts[1:])}
-    return {"rows": out, "source": str(path.relative_to(ROOT))}
+    if key != kernel_key():
+        return None, f"{path.name} holds counters of other code (key {key}, this code's is {kernel_key()})"
+    return {"rows": out, "source": f"profiles/{path.name}"}, None
+
+
+def counter_fractions(cs, avg_s, step_s):
+    """What a counter table says beside this run's times: HBM bytes per sweep
+    launch, their share of the HBM peak, the sweeps' VALU share and its
+    column, and the whole path's share of the HBM peak; the entries a table
+    lacks are None.  A share above 1 is none: then nothing is taken from the
+    table, and the reason comes with it."""
+    none = dict(traffic=None, hbm=None, valu=None, column=None, path=None)
+    if cs is None:
+        return none, None
+    frows = [v for k, v in cs["rows"].items() if k.startswith("k_flux<")]
+    out = dict(none)
+    peak = HBM_PEAK_GBS * 1e9
+    if frows and all(r.get("hbm_MB") is not None for r in frows):
+        launches = sum(r["per_step"] for r in frows)
+        out["traffic"] = sum(r["hbm_MB"] * r["per_step"] for r in frows) / launches * 1e6
+        out["hbm"] = out["traffic"] / avg_s / peak
+    # VALU issue fraction (wave64 VALU instructions x 4 cycles over the SIMD
+    # cycles of the launch), else the SQ_ACTIVE_INST_VALU busy fraction
+    for col in ("valu_issue", "valu_busy"):
+        if out["valu"] is None and frows and all(r.get(col) is not None for r in frows):
+            us = sum(r["avg_us"] * r["per_step"] for r in frows)
+            out["valu"] = sum(r[col] * r["avg_us"] * r["per_step"] for r in frows) / us
+            out["column"] = col
+    if all(r.get("hbm_MB") is not None for r in cs["rows"].values()):
+        out["path"] = sum(r["hbm_MB"] * 1e6 * r["per_step"] for r in cs["rows"].values()) / step_s / peak
+    for name in ("hbm", "valu", "path"):
+        if out[name] is not None and out[name] > 1.0:
+            return none, f"{cs['source']}: {name} share {out[name]:.2f} of this run's time is above 1"
+    return out, None
 
 
 def profile_form(args, prob, forms):
@@ -478,16 +533,13 @@ def main():
     alg_tfs = fl_flops / (fl_ms * 1e-3) / 1e12
     # counters of the timed plain-form dispatches (committed summary, see
     # --summarize): HBM bytes per launch and VALU busy of the k_flux family
-    cs = read_counter_summary(args.workload, "plain_fp64")
-    frows = [v for k, v in cs["rows"].items() if k.startswith("k_flux<")] if cs else []
-    traffic = (sum(r["hbm_MB"] for r in frows) / len(frows) * 1e6
-               if frows and all(r.get("hbm_MB") is not None for r in frows) else None)
-    # VALU issue fraction (wave64 VALU instructions x 4 cycles over the SIMD
-    # cycles of the launch), else the SQ_ACTIVE_INST_VALU busy fraction
-    col = "valu_issue" if frows and all(r.get("valu_issue") is not None for r in frows) else "valu_busy"
-    busy = (sum(r[col] for r in frows) / len(frows)
-            if frows and all(r.get(col) is not None for r in frows) else None)
-    hbm_counter_frac = traffic / avg_s / (HBM_PEAK_GBS * 1e9) if traffic else None
+    cs, refused = read_counter_summary(args.workload, "plain_fp64")
+    counters, above = counter_fractions(cs, avg_s, el / args.steps)
+    refused = refused or above
+    traffic, hbm_counter_frac = counters["traffic"], counters["hbm"]
+    busy, col = counters["valu"], counters["column"]
+    if refused:
+        note(f"counters not used: {refused}")
     # the binding roof: the counters' VALU busy against their HBM fraction;
     # without counters, the algorithmic intensity against the FP64 ridge
     if busy is not None and hbm_counter_frac is not None:
@@ -503,7 +555,8 @@ def main():
         "unit": "TFLOP/s" if bound == "valu" else "GB/s",
         "frac": round(alg_tfs / FP64_PEAK_TFS if bound == "valu" else alg_gbs / HBM_PEAK_GBS, 4),
         "traffic": round(traffic) if traffic else None,
-        "traffic_source": cs["source"] if cs else None,
+        "traffic_source": cs["source"] if traffic else None,
+        "counters_not_used": refused,
         "avg_launch_ms": round(avg_s * 1e3, 4),
         "alg_bytes_per_launch": round(fl_bytes / max(1, fl_launch)),
         "alg_flops_per_launch": round(fl_flops / max(1, fl_launch)),
@@ -518,10 +571,7 @@ def main():
     b_alg = 8.0 * (48 + 8 * prob.cfg.get("nscalars", 0))
     # the plain path's counter HBM fraction: every kernel's committed bytes per
     # dispatch times its dispatches per step, over this run's time per step
-    path_counter = None
-    if cs and all(r.get("hbm_MB") is not None for r in cs["rows"].values()):
-        step_hbm = sum(r["hbm_MB"] * 1e6 * r["per_step"] for r in cs["rows"].values())
-        path_counter = step_hbm / (el / args.steps) / (HBM_PEAK_GBS * 1e9)
+    path_counter = counters["path"]
     line = {
         "metric": METRIC,
         "value": round(value, 1),
