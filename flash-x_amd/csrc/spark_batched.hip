@@ -1,12 +1,11 @@
-// spark_batched.hip -- the batched form of the Spark RK stage: one fused,
-// persistent launch per RK stage over every block of the batch.
-//
-// This is the FP32-flux form: FP32 reconstruction and Riemann arithmetic
-// (built with -ffp-contract=fast); conserved-variable accumulation, floors,
-// EOS and flux-register sums are FP64.  (The same kernel in FP64 needed ~330
-// registers, one wave per SIMD: 8 steps of 360 leaves of 16^3 with 8 scalars on
-// three levels took 65 ms against 33 ms in the directional sweeps of
-// spark_plain.hip, which run the batched FP64 form instead.)
+// spark_batched.hip -- the FP32-flux form of the Spark RK stage: one fused,
+// persistent launch per RK stage over every block of the batch, FP32
+// reconstruction and Riemann arithmetic (built with -ffp-contract=fast);
+// conserved-variable accumulation, floors, EOS and flux-register sums are
+// FP64.  (The same kernel in FP64 needed ~330 registers, one wave per SIMD: 8
+// steps of 360 leaves of 16^3 with 8 scalars on three levels took 65 ms against
+// 33 ms in the directional sweeps of spark_plain.hip, which run the batched
+// FP64 form instead.)
 //
 // Work items are (block, x-y tile); a workgroup takes items from per-XCD
 // queues (an XCD's queue holds whole blocks, so the halos that tiles of one
@@ -39,8 +38,9 @@ namespace {
 
 using Real = float;
 constexpr int NT = FUSED_THREADS;
-// hydro slots staged per cell: dens velx vely velz pres rhoe.  The form takes gamc = gamma (the Gamma EOS sets every cell's gamc to
-// gamma), so it neither stages nor reconstructs it.
+// hydro slots staged per cell: dens velx vely velz pres rhoe.  The form takes
+// gamc = gamma (the Gamma EOS sets every cell's gamc to gamma), so it neither
+// stages nor reconstructs it.
 constexpr int NH = 6;
 constexpr int CH = FUSED_SCALAR_CHUNK;  // mass scalars per chunk (the species all in the first)
 constexpr int SL_RHOE = NH - 1;

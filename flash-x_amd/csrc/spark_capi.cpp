@@ -108,7 +108,7 @@ struct spark_batch {
   bool batched = false;
   int cus = 0;            // compute units of the device
   size_t lds_limit = 0;   // LDS bytes a workgroup may allocate
-  int64_t* nbr_d = nullptr;  // uniform grid: 27 neighbour pool offsets per block
+  int64_t* nbr_d = nullptr;  // 27 neighbour pool offsets per block (uniform grid, hierarchy)
   bool amr = false;          // block hierarchy declared (spark_set_amr_grid)
   // block hierarchy: blocks that compute no guard sector read all their halo
   // from leaves around them (nbr_d row), every stage over the interior only
@@ -140,7 +140,7 @@ struct spark_batch {
   bool dt_control = false;
   int amr_remap_count = 0;
   int amr_partial_count = 0;
-  // plain form on a block hierarchy: per stage the boxes its sweeps run, one
+  // FP64 forms on a block hierarchy: per stage the boxes the sweeps run, one
   // group per box shape (plain_groups_build)
   struct PlainGroup {
     int ext[3];
@@ -243,8 +243,8 @@ int required_guard(const spark_params& p) {
   double c[3][3], w[3];
   rk_tables(p, &last, c, la, w);
   const int maxoff = (p.guard_mode == SPARK_GUARD_REFILL) ? 0 : la[0];
-  // the fused kernel of the batched forms stages a 3-cell halo whatever
-  // the reconstruction's own stencil
+  // the FP32-flux form's kernel stages a 3-cell halo whatever the
+  // reconstruction's own stencil (both batched forms ask for it)
   const bool fused = p.form == SPARK_FORM_FP32_FLUX || p.form == SPARK_FORM_BATCHED_FP64;
   return maxoff + (fused ? std::max(p.nstencil, 3) : p.nstencil);
 }
@@ -434,9 +434,9 @@ int run_step_begin(spark_batch* b, bool same_level, bool last) {
   // outer layers are never read before the next refill).  Without the
   // hybrid solver no form reads SHOK, so it is computed for the interior,
   // where it is part of the solution; guard-layer SHOK, which only the
-  // hybrid solver reads, is left as it was.  The batched forms read SHOK
-  // from the block's own box, so remapping blocks (no guard cells of their
-  // own in the stages) get it one layer out.
+  // hybrid solver reads, is left as it was.  The stages read SHOK from the
+  // block's own box, so remapping blocks (no guard cells of their own in the
+  // stages) get it one layer out.
   const bool hyb = b->p.use_hybrid_riemann != 0;
   const int band = !hyb ? 0 : (b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[0]) + 1;
   if (amr_remap_on(b) && (b->batched || (same_level && !last))) {
@@ -493,7 +493,7 @@ int stage_ngoff(const spark_batch* b, int stage) {
   return b->p.guard_mode == SPARK_GUARD_REFILL ? 0 : b->limits_array[stage - 1];
 }
 
-// stage region of one block in the batched forms: blocks that read all
+// stage region of one block in the FP32-flux form: blocks that read all
 // their halos from same-level neighbours update only their interior (the
 // region of a block that reads some is built by partial_boxes())
 int blk_ngoff(const spark_batch* b, int blk, int stage) {
@@ -931,7 +931,7 @@ int fused_plan(spark_batch* b) {
   return SPARK_OK;
 }
 
-// The plain form's stage boxes on a hierarchy.  Every block's interior is one
+// The FP64 forms' stage boxes on a hierarchy.  Every block's interior is one
 // group (full telescoping boxes of the blocks without a same-level leaf
 // around are another); the computed sectors of the others beside it are a
 // group per box shape.  Blocks share few sector masks, so a mask's boxes are

@@ -1,7 +1,9 @@
-// spark_plain.hip -- the plain FP64 form of the Spark RK stage on gfx950.
+// spark_plain.hip -- the Spark RK stage in FP64 on gfx950 (plain and batched
+// FP64 forms).
 //
 // One launch per kernel per stage over all blocks of one shape (blockIdx.y
-// walks the block list).  The dataflow follows the reference per stage
+// walks the block list), on a hierarchy one per box shape of the stage
+// region.  The dataflow follows the reference per stage
 // (Spark/Hydro.F90-mc:144-194): flattening -> face fluxes per direction ->
 // conserved update + floors + Gamma EOS.  Each sweep turns its face fluxes
 // into its term of the update's flux divergence per cell (the x sweep
@@ -690,10 +692,10 @@ __global__ void __launch_bounds__(256) k_shock(DevParams P, const BlockMeta* __r
 // LDS, so every value is loaded once and the sound speed computed once per
 // cell.  Cells of the band box get the flag, the outer layer 0, as the
 // two-pass kernels above give.  Tiles are as wide as the box up to SHK_T
-// per side.  NB: cells outside the interior are read through a neighbour
-// table (nbr: 27 pool offsets per block, no guard sector its own) from the
-// leaf) from the leaves around the block, so its own guard cells need no
-// fill; the flags are still written into the block's own box.
+// per side.  NB: cells outside the interior are read through the neighbour
+// table (nbr: 27 pool offsets per block, no guard sector computed by the block
+// itself) from the blocks around it, so its own guard cells need no fill; the
+// flags are still written into the block's own box.
 constexpr int SHK_T = 20;
 constexpr int SHK_GROUPS = 1536;
 constexpr int SHK_F = 5;  // staged fields: pres, sound speed, velx, vely, velz

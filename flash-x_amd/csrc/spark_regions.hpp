@@ -119,7 +119,7 @@ inline void sector_boxes(int nx, int ny, int nz, int g, int e, uint32_t local, s
 
 // The computed sectors alone, without the interior, as disjoint boxes: the
 // largest union of sectors that is a box first (in sectors; 0 and +-1 per
-// dimension have at most 6 ranges), until none is left.  The plain form's
+// dimension have at most 6 ranges), until none is left.  The FP64 forms'
 // sweeps run every block's interior in one launch and these boxes in one
 // launch per box shape, so few large boxes count; a level change across one
 // face gives one slab.
