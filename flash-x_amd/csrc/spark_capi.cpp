@@ -82,10 +82,11 @@ struct spark_batch {
   std::vector<BlockMeta> meta_h;
   BlockMeta* meta_d = nullptr;
   std::vector<ShapeClass> classes;
-  int64_t pool = 0, opool = 0, bpool = 0;  // sizes in doubles
+  int64_t pool = 0, opool = 0, dpool = 0, bpool = 0;  // sizes in doubles
   double* U = nullptr;
   double* S = nullptr;
   double* flat = nullptr;
+  double* div = nullptr;  // FP64 forms, where memory allows: the sweeps' divergence terms per cell
   double* fb[3] = {nullptr, nullptr, nullptr};
   double* dtp = nullptr;
   long long* loc = nullptr;
@@ -228,7 +229,7 @@ PlainLaunch make_launch(spark_batch* b, const ShapeClass& c) {
   L.Sin = b->S;
   L.Sout = b->S;
   L.flat = b->flat;
-  L.div = nullptr;
+  L.div = spark::DivTerms{nullptr, 0};
   for (int d = 0; d < 3; d++) L.fb[d] = b->p.flux_correct ? b->fb[d] : nullptr;
   L.weight = 0.;
   L.add_flux = 0;
@@ -251,6 +252,14 @@ int required_guard(const spark_params& p) {
 
 bool ug_remap(const spark_batch* b);
 void drop_graph(spark_batch* b);
+
+// memory of the current device that is free for certain: the runtime counts up
+// to half a GiB more than it can allocate
+int64_t free_memory() {
+  size_t free_bytes = 0, total = 0;
+  if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) return 0;
+  return std::max<int64_t>(0, (int64_t)free_bytes - (int64_t(1) << 30));
+}
 
 // a host vector on the device (the caller frees it)
 template <class T> hipError_t upload(T** dst, const std::vector<T>& v) {
@@ -479,14 +488,13 @@ double* stage_out(spark_batch* b, int stage) {
   return stage == 1 ? b->S : b->S2;
 }
 
-// where the sweeps of a stage keep their divergence terms: the stage's own
-// output, and in the last stage, which writes the solution its update reads,
-// the buffer that stage does not use (S is not read again after stage 2 of RK3,
-// RK2 has no stage 2 buffer).  A pool of their own (5 + N_s fields) would take a
-// fifth more memory than the state.
-double* stage_div(spark_batch* b, int stage) {
-  if (stage != b->last_stage) return stage_out(b, stage);
-  return b->last_stage == 3 ? b->S : b->S2;
+// where the sweeps of a stage keep their divergence terms: their own pool, or
+// the stage's output and, in the last stage, which writes the solution its
+// update reads, the buffer that stage does not use (S is not read again after
+// stage 2 of RK3, RK2 has no stage 2 buffer)
+spark::DivTerms stage_div(spark_batch* b, int stage) {
+  if (b->div) return spark::DivTerms{b->div, 0};
+  return spark::DivTerms{stage != b->last_stage ? stage_out(b, stage) : b->last_stage == 3 ? b->S : b->S2, spark::DIV_SKIP};
 }
 
 int stage_ngoff(const spark_batch* b, int stage) {
@@ -693,6 +701,7 @@ void free_batch(spark_batch* b) {
   F(b->meta_d);
   for (auto& c : b->classes) F(c.ids_d);
   F(b->U); F(b->S); F(b->flat);
+  F(b->div);
   for (int d = 0; d < 3; d++) F(b->fb[d]);
   F(b->dtp); F(b->loc); F(b->dt_hist); F(b->dtparts); F(b->err);
   delete b;
@@ -1134,15 +1143,13 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
 
   const int g = p->nguard;
   const int nf = 5 + p->nscalars;
-  size_t free_bytes = 0, total_bytes = 0;
-  if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) free_bytes = 0;
   int64_t padded = 0;
   for (int i = 0; i < nblocks; i++) {
     const int NX = blocks[i].nx + 2 * g;
     padded += (int64_t)spark::row_pad(NX, g).pitch * (p->ndim > 1 ? blocks[i].ny + 2 * g : 1) *
               (p->ndim > 2 ? blocks[i].nz + 2 * g : 1);
   }
-  const bool pad_rows = spark::pad_rows(padded, 3 * nvar + 1, (int64_t)free_bytes);
+  const bool pad_rows = spark::pad_rows(padded, 3 * nvar + 1, free_memory());
   std::map<std::tuple<int, int, int>, int> cls;
   int64_t max_int = 0;
   for (int i = 0; i < nblocks; i++) {
@@ -1166,6 +1173,8 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
     b->pool += (int64_t)nvar * m.cstride;
     m.obase = b->opool + rp.lead;
     b->opool += m.cstride;
+    m.dbase = b->dpool + rp.lead;
+    b->dpool += (int64_t)nf * m.cstride;
     int64_t reg = 1;
     for (int q = 0; q < 3; q++) reg *= n[q] + (q < p->ndim ? 1 : 0);
     m.bbase = b->bpool;
@@ -1233,6 +1242,14 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
     ALLOC(b->tune_err, sizeof(int));
     ALLOC(b->tune_dt, sizeof(double));
   }
+  // last, from what the batch leaves (1D has no sweep before the last)
+  if (p->form != SPARK_FORM_FP32_FLUX && p->ndim > 1) {
+    if (spark::div_pool(b->dpool, free_memory()) &&
+        hipMalloc((void**)&b->div, sizeof(double) * b->dpool) != hipSuccess) {
+      (void)hipGetLastError();  // the stage buffers serve
+      b->div = nullptr;
+    }
+  }
 #undef ALLOC
   HIPCHK(hipMemcpyAsync(b->meta_d, b->meta_h.data(), sizeof(BlockMeta) * nblocks, hipMemcpyHostToDevice, g_stream));
   for (auto& c : b->classes)
@@ -1241,6 +1258,7 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   HIPCHK(hipMemsetAsync(b->S, 0, sizeof(double) * b->pool, g_stream));
   HIPCHK(hipMemsetAsync(b->flat, 0, sizeof(double) * b->opool, g_stream));
   HIPCHK(hipMemsetAsync(b->S2, 0, sizeof(double) * b->pool, g_stream));
+  if (b->div) HIPCHK(hipMemsetAsync(b->div, 0, sizeof(double) * b->dpool, g_stream));
   if (p->flux_correct)
     for (int q = 0; q < 3; q++) HIPCHK(hipMemsetAsync(b->fb[q], 0, sizeof(double) * b->bpool, g_stream));
   HIPCHK(hipMemsetAsync(b->err, 0, sizeof(int), g_stream));

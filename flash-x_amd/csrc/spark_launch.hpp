@@ -46,6 +46,20 @@ __device__ __forceinline__ int64_t box_cell(const BlockMeta& m, int64_t t) {
   return t + row * (m.PX - m.NX);
 }
 
+// Where a stage's sweeps keep their divergence terms: a pool of 5 + ns fields
+// (skip = 0: term n in field n at BlockMeta::dbase) or a state buffer (skip =
+// DIV_SKIP, at BlockMeta::base), there in fields that the stage's update writes
+// (dens, eint, vel(3), the scalars), so that the buffer may be the stage's own
+// output: the update reads every term of a cell before it writes the field that
+// holds it.
+struct DivTerms {
+  double* p;
+  int skip;
+};
+constexpr int DIV_SKIP = V_VELX - 2;
+static_assert(V_DENS == 0 && V_EINT == 1 && V_VELY == V_VELX + 1 && V_VELZ == V_VELX + 2 && V_NPROP == F_NUM + DIV_SKIP,
+              "the terms' fields are the ones the update writes");
+
 // Everything one plain-form launch sequence needs for a list of blocks that
 // share one interior shape.
 struct PlainLaunch {
@@ -66,7 +80,7 @@ struct PlainLaunch {
   const double* Sin;      // stage input state (U at stage 1, S after)
   double* Sout;           // stage output state (U at the last stage, S before)
   double* flat;           // flattening coefficients / scratch (cell pool)
-  double* div;            // state buffer holding the divergence terms of the sweeps so far (2D, 3D)
+  DivTerms div;           // divergence terms of the sweeps so far (2D, 3D)
   double* fb[3];          // flux-register pools (nullptr when not correcting)
   double weight;          // flux-register weight of this stage
   int add_flux;           // 0: overwrite (stage 1), 1: accumulate

@@ -306,20 +306,11 @@ __device__ __forceinline__ void update_cell(const DevParams& P, const BlockMeta&
   }
 }
 
-// Field of a state buffer that holds flux n's divergence term while a stage
-// runs: one the stage's update writes (dens, eint, vel(3), the scalars), so that
-// the buffer may be the stage's own output.  update_cell reads every term of a
-// cell before it writes the field that holds it.
-__device__ __forceinline__ int div_field(int n) { return n < 2 ? n : n + V_VELX - 2; }
-static_assert(V_DENS == 0 && V_EINT == 1 && V_VELY == V_VELX + 1 && V_VELZ == V_VELX + 2 &&
-                  V_NPROP == V_VELX - 2 + F_NUM,
-              "div_field: the terms' fields are the ones the update writes");
-
 // what a sweep needs for its part of the stage update
 struct UpdArgs {
   const double* U0;  // step input (U); may alias Sout
   double* Sout;      // stage output state
-  double* div;       // state buffer that holds the divergence terms of the sweeps so far (div_field)
+  DivTerms div;      // the divergence terms of the sweeps so far (5 + ns per cell)
   const double* dtp;
   double c1, c2, c3;
   int final_stage;
@@ -597,7 +588,8 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
   const double dd = DIR == 0 ? m.dx : DIR == 1 ? m.dy : m.dz;
   double facM = 1.0, facP = 1.0, rc = 0.0;
   if (DIR == 0) (void)geo_facs(P, m.id, ijk[0], ijk[1], m.dx, facM, facP, rc);
-  double* dv = UA.div + m.base + c;
+  double* dv = UA.div.p + (UA.div.skip ? m.base : m.dbase) + c;
+  auto div_field = [&](int n) -> int64_t { return (n < 2 ? n : n + UA.div.skip) * m.cstride; };
   // flux n's term, added to the earlier directions' (prev) as the update
   // writes it: -(dt/dx (facP F+ - facM F-)), then - dt/dy (G+ - G-), ...
   auto term = [&](int n, double prev) -> double {
@@ -606,7 +598,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
     return prev - dt / dd * (hi - lo);
   };
   if (STEP == 3) {
-    auto inner_of = [&](int n) -> double { return term(n, DIR == 0 ? 0.0 : dv[div_field(n) * m.cstride]); };
+    auto inner_of = [&](int n) -> double { return term(n, DIR == 0 ? 0.0 : dv[div_field(n)]); };
     update_cell<NSM>(P, m, ijk[0], ijk[1], c, UA.U0 + m.base, sp, UA.Sout + m.base, inner_of, dt, UA.c1, UA.c2,
                      UA.c3, UA.final_stage);
   } else {
@@ -614,10 +606,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(STEP 
     // F_NUM + ns re-reads the last)
     double prev[NFM];
 #pragma unroll
-    for (int n = 0; n < NFM; n++) prev[n] = STEP == 2 ? dv[div_field(n < F_NUM + ns ? n : F_NUM + ns - 1) * m.cstride] : 0.0;
+    for (int n = 0; n < NFM; n++) prev[n] = STEP == 2 ? dv[div_field(n < F_NUM + ns ? n : F_NUM + ns - 1)] : 0.0;
 #pragma unroll
     for (int n = 0; n < NFM; n++)
-      if (n < F_NUM + ns) dv[div_field(n) * m.cstride] = term(n, prev[n]);
+      if (n < F_NUM + ns) dv[div_field(n)] = term(n, prev[n]);
   }
 }
 

@@ -35,4 +35,13 @@ inline bool pad_rows(int64_t cells, int64_t fields, int64_t free_bytes) {
   return cells * fields * (int64_t)sizeof(double) <= free_bytes / 8 * 3;
 }
 
+// Whether the FP64 sweeps get a pool of their own for their divergence terms:
+// where it takes no more than a quarter of the memory its batch leaves.  Without
+// it they keep the terms in the stage buffers, which is as fast for most
+// batches; on 4384 leaves of 16^3 with 8 scalars the x sweep, then writing the
+// buffer beside the one it reads, takes 13.8 instead of 11.3 ms a step.
+inline bool div_pool(int64_t doubles, int64_t free_bytes) {
+  return doubles * (int64_t)sizeof(double) <= free_bytes / 4;
+}
+
 }  // namespace spark

@@ -119,7 +119,8 @@ int spark_finalize(void);
  * (the reference allocates scratch per block; here once per batch).  Three
  * states of 11 + N_s doubles per guard-celled cell and one field; rows are
  * padded to memory lines (a third more at most) where the padded states take
- * no more than 3/8 of the device memory that is free. */
+ * no more than 3/8 of the device memory that is free, and the FP64 forms hold
+ * 5 + N_s fields more where those take no more than a quarter of what is left. */
 int spark_batch_create(const spark_params* p, int nblocks, const spark_block_desc* blocks, spark_batch** out);
 int spark_batch_destroy(spark_batch* b);
 

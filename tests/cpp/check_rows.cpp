@@ -2,7 +2,8 @@
 // interior cell of every row starts a line or half line of 128 bytes, rows
 // hold their cells, at most a third more memory), and pad_rows: a padded
 // state fits into the memory that is free, also for widths whose padding is
-// small, and takes at most 3/32 of it from the batches after it.  Prints "ok <cases>" or the first mismatch.
+// small, and takes at most 3/32 of it from the batches after it; div_pool
+// likewise.  Prints "ok <cases>" or the first mismatch.
 #include <cstdio>
 
 #include "spark_rows.hpp"
@@ -32,6 +33,11 @@ int main() {
         }
         if (!pad && free == 4 * packed) {
           std::printf("width %d guards %d: not padded in four times its memory\n", nx, ng);
+          return 1;
+        }
+        const int64_t left = free - (pad ? padded : packed), pool = rows * (pad ? p.pitch : NX) * 13;
+        if (spark::div_pool(pool, left) && pool * 8 > left / 4) {
+          std::printf("width %d guards %d: a pool of %lld doubles in %lld bytes\n", nx, ng, (long long)pool, (long long)left);
           return 1;
         }
         cases++;
