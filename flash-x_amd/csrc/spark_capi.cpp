@@ -272,7 +272,7 @@ template <class T> hipError_t upload(T** dst, const std::vector<T>& v) {
 // computes only its interior and the other sectors.  The values are those of
 // telescoping (the same cells from the same inputs).
 bool amr_remap_on(const spark_batch* b) {
-  return b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
+  return b->amr && b->same_level && b->amr_remap_count + b->amr_partial_count > 0;
 }
 
 void free_amr_fill(spark_batch* b) {
@@ -1822,6 +1822,10 @@ int spark_set_amr_grid(spark_batch* b, int nbx0, int nby0, int nbz0, const int* 
   // this gives are those of telescoping: the same cells from the same
   // inputs, since the guard fill is a function of the cell's position and
   // the leaves' data.
+  // (from here on a failed allocation leaves a batch without a hierarchy)
+  b->amr = false;
+  b->planned = false;
+  drop_graph(b);
   b->amr_remap_blk.assign(b->nblk, 0);
   b->amr_local.assign(b->nblk, 0);
   b->amr_remap_count = 0;
