@@ -145,8 +145,10 @@ __device__ __forceinline__ double rcp_in_range(double b) {
 // quotient underflows adds nothing to 1).  The products by 2, 4 and 0.25 are
 // exact (0.25 s^2 underflows only where the 1e-36 swamps it), so fusing them
 // with the addition that follows rounds the same: 8 fewer instructions.
-// Otherwise, NaN and infinities included, the wave takes the expressions above
-// as they stand.  Sweeps of 576 blocks of 16^3 with 8 scalars,
+// Otherwise, NaN and infinities included, the wave takes weno5 whole, in one
+// branch out of the way of the others' code (divides in branches of their own
+// between the weights: 2D tube of 16 blocks of 16^2 355 -> 364 us a pass, 64
+// blocks of 16^3 4.01 -> 4.09 ms).  Sweeps of 576 blocks of 16^3 with 8 scalars,
 // telescoping: x 2.87 -> 2.65, y 3.39 -> 3.29, z 4.56 -> 4.44 ms per step.
 // (One range test after all variables, and the whole reconstruction again
 // where it fails, spills and measured 2.79 / 3.38 / 4.55.)
@@ -160,40 +162,20 @@ __device__ __forceinline__ void weno5_short(double um2, double um1, double u0, d
   const double s1 = __builtin_fma(-4., um1, um2) + u03;
   const double s2 = um1 - up1;
   const double s3 = __builtin_fma(-4., up1, u03) + up2;
-  double b1 = __builtin_fma(0.25, s1 * s1, n13o12 * (t1 * t1));
-  double b2 = __builtin_fma(0.25, s2 * s2, n13o12 * (t2 * t2));
-  double b3 = __builtin_fma(0.25, s3 * s3, n13o12 * (t3 * t3));
-  const bool in_range = __ballot(!(__builtin_fma(u0, u0, b1) + b3 < 0x1p900)) == 0;
-  double r1, r2, r3;
-  if (in_range) {
-    const double tau = __builtin_fabs(b1 - b3);
-    r1 = div_in_range(tau, b1 + eps);
-    r2 = div_in_range(tau, b2 + eps);
-    r3 = div_in_range(tau, b3 + eps);
-  } else {
-    auto beta = [&](double t, double s) { return n13o12 * (t * t) + 0.25 * (s * s); };
-    b1 = beta(um2 - 2. * um1 + u0, um2 - 4. * um1 + 3. * u0);
-    b2 = beta(um1 - 2. * u0 + up1, um1 - up1);
-    b3 = beta(u0 - 2. * up1 + up2, 3. * u0 - 4. * up1 + up2);
-    const double tau = __builtin_fabs(b1 - b3);
-    r1 = tau / (b1 + eps);
-    r2 = tau / (b2 + eps);
-    r3 = tau / (b3 + eps);
+  const double b1 = __builtin_fma(0.25, s1 * s1, n13o12 * (t1 * t1));
+  const double b2 = __builtin_fma(0.25, s2 * s2, n13o12 * (t2 * t2));
+  const double b3 = __builtin_fma(0.25, s3 * s3, n13o12 * (t3 * t3));
+  if (__builtin_expect(__ballot(!(__builtin_fma(u0, u0, b1) + b3 < 0x1p900)) != 0, 0)) {
+    weno5<double>(um2, um1, u0, up1, up2, flat, oup, oum);
+    return;
   }
-  r1 = 1. + r1;
-  r2 = 1. + r2;
-  r3 = 1. + r3;
+  const double tau = __builtin_fabs(b1 - b3);
+  const double r1 = 1. + div_in_range(tau, b1 + eps);
+  const double r2 = 1. + div_in_range(tau, b2 + eps);
+  const double r3 = 1. + div_in_range(tau, b3 + eps);
   const double A1 = 0.1 * r1, A2 = 0.6 * r2, A3 = 0.3 * r3;
   const double M1 = 0.3 * r1, M3 = 0.1 * r3;
-  const double As = A1 + A2 + A3, Ms = M1 + A2 + M3;
-  double ia, im;
-  if (in_range) {
-    ia = rcp_in_range(As);
-    im = rcp_in_range(Ms);
-  } else {
-    ia = 1. / As;
-    im = 1. / Ms;
-  }
+  const double ia = rcp_in_range(A1 + A2 + A3), im = rcp_in_range(M1 + A2 + M3);
   const double W5p1 = 2. / 6. * um2 + -7. / 6. * um1 + 11. / 6. * u0;
   const double W5p2 = -1. / 6. * um1 + 5. / 6. * u0 + 2. / 6. * up1;
   const double W5p3 = 2. / 6. * u0 + 5. / 6. * up1 + -1. / 6. * up2;
