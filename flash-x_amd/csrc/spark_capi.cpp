@@ -56,11 +56,15 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
+// a failure is reported once: what the runtime keeps of it would come back as
+// the error of the next launch
 #define HIPCHK(expr)                                                                           \
   do {                                                                                         \
     hipError_t e_ = (expr);                                                                    \
-    if (e_ != hipSuccess) return fail(SPARK_ERR_HIP, "%s: %s (%s:%d)", #expr, hipGetErrorString(e_), \
-                                      __FILE__, __LINE__);                                     \
+    if (e_ != hipSuccess) {                                                                    \
+      (void)hipGetLastError();                                                                 \
+      return fail(SPARK_ERR_HIP, "%s: %s (%s:%d)", #expr, hipGetErrorString(e_), __FILE__, __LINE__); \
+    }                                                                                          \
   } while (0)
 
 inline int64_t round_up(int64_t a, int64_t m) { return (a + m - 1) / m * m; }
@@ -1203,6 +1207,7 @@ int spark_batch_create(const spark_params* p, int nblocks, const spark_block_des
   do {                                                                                 \
     hipError_t e_ = hipMalloc((void**)&(ptr), (bytes));                                \
     if (e_ != hipSuccess) {                                                            \
+      (void)hipGetLastError();                                                         \
       free_batch(b);                                                                   \
       return fail(SPARK_ERR_HIP, "hipMalloc(%zu bytes): %s", (size_t)(bytes), hipGetErrorString(e_)); \
     }                                                                                  \

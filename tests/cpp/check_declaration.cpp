@@ -2,9 +2,10 @@
 // runs as one without a hierarchy: the C API is built on stand-ins of the HIP
 // runtime and of the kernels' launch functions (host memory, nothing runs), and
 // each device allocation of spark_set_amr_grid fails in turn, in a first
-// declaration and in one over an earlier hierarchy.  Every pointer that a launch
-// is handed has to be an allocation that is still there.  Prints "ok <cases>"
-// or the first mismatch.
+// declaration and in one over an earlier hierarchy; so does each allocation of
+// spark_batch_create before it.  Every pointer that a launch is handed has to be
+// an allocation that is still there, and no launch returns the error of a call
+// before it.  Prints "ok <cases>" or the first mismatch.
 #include "../../flash-x_amd/csrc/spark_capi.cpp"
 
 #include <cstdlib>
@@ -16,6 +17,7 @@ int fail_at = -1;  // the allocation that fails (counted down), < 0: none
 int allocations = 0;
 int fills = 0, table_reads = 0, stages = 0;
 bool bad = false;
+hipError_t kept = hipSuccess;  // what hipGetLastError returns once, as after a launch
 
 void expect(bool ok, const char* what) {
   if (!ok && !bad) std::printf("%s\n", what);
@@ -42,7 +44,7 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
   allocations++;
   *p = nullptr;
-  if (fail_at >= 0 && fail_at-- == 0) return hipErrorOutOfMemory;
+  if (fail_at >= 0 && fail_at-- == 0) return kept = hipErrorOutOfMemory;
   *p = std::calloc(1, std::max<size_t>(1, n));
   live[*p] = n;
   return hipSuccess;
@@ -66,7 +68,11 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)1; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = kept;
+  kept = hipSuccess;
+  return e;
+}
 const char* hipGetErrorString(hipError_t) { return "an error"; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)1; return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -87,7 +93,7 @@ hipError_t plain_stage(const PlainLaunch& L, int, double, double, double, int) {
   check(L);
   expect(allocated(L.Sin) && allocated(L.Sout) && allocated(L.div.p), "a stage without its states");
   stages++;
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t plain_shock_detect(const PlainLaunch& L, double*, double*, int, const int64_t* nbr) {
   check(L);
@@ -95,7 +101,10 @@ hipError_t plain_shock_detect(const PlainLaunch& L, double*, double*, int, const
   table_reads += nbr != nullptr;
   return hipSuccess;
 }
-hipError_t plain_set_scalar(hipStream_t, double* p, double) { expect(allocated(p), "no dt"); return hipSuccess; }
+hipError_t plain_set_scalar(hipStream_t, double* p, double) {
+  expect(allocated(p), "no dt");
+  return hipGetLastError();
+}
 hipError_t plain_correct(const PlainLaunch& L, double*, const unsigned char* f) {
   check(L);
   expect(!f || allocated(f), "face masks that are not there");
@@ -126,7 +135,7 @@ hipError_t fused_stage(const FusedArgs& A, int, size_t, hipStream_t) {
   expect(allocated(A.Sin) && allocated(A.Sout) && (!A.nbr || allocated(A.nbr)), "a fused stage without its tables");
   table_reads += A.nbr != nullptr;
   stages++;
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t noalloc_scratch_address(void** p) { *p = (void*)256; return hipSuccess; }
 void xfer_release() {}
@@ -181,6 +190,24 @@ int main() {
   int cases = 0;
   if (spark_init(0) != SPARK_OK) return std::printf("spark_init\n"), 1;
   std::vector<int> org;
+  for (int form : {SPARK_FORM_PLAIN_FP64, SPARK_FORM_BATCHED_FP64, SPARK_FORM_FP32_FLUX})
+    for (int k = 0;; k++, cases++) {
+      // the pool of the divergence terms is left out where it cannot be had
+      const size_t before = live.size();
+      fail_at = k;
+      spark_batch* b = make(form, org);
+      const bool failed = fail_at < 0;
+      fail_at = -1;
+      expect(kept == hipSuccess, "an error that is kept");
+      if (!b) {
+        expect(failed && live.size() == before, "a batch that failed holds memory");
+        continue;
+      }
+      expect(spark_hydro_step(b, 1e-3, 1e-3) == SPARK_OK, "a step that fails");
+      spark_batch_destroy(b);
+      if (bad) return std::printf("form %d, allocation %d of a batch\n", form, k), 1;
+      if (!failed) break;
+    }
   for (int form : {SPARK_FORM_PLAIN_FP64, SPARK_FORM_BATCHED_FP64, SPARK_FORM_FP32_FLUX})
     for (bool over : {false, true}) {
       auto declare = [&](spark_batch* b) { return spark_set_amr_grid(b, 2, 1, 2, org.data(), bc); };
