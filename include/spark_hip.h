@@ -195,7 +195,9 @@ int spark_set_uniform_grid(spark_batch* b, int nbx, int nby, int nbz);
  * spark_fill_guardcells goes before them.  With flux_correct the
  * FP32-flux form corrects only the cells on faces toward a finer leaf (the
  * correction is zero elsewhere; the FP64 forms still pass those cells
- * through the reference's conserved/primitive round trip).
+ * through the reference's conserved/primitive round trip).  A declaration
+ * that returns SPARK_ERR_HIP (no memory for its tables) leaves the batch
+ * without a hierarchy; it may be declared again.
  * Replaces: Grid_fillGuardCells over PARAMESH leaves,
  * Grid/GridMain/AMR/Paramesh4/Grid_fillGuardCells.F90:436-546, and the
  * flux hand-off of Spark/Hydro.F90-mc:197-236. */
